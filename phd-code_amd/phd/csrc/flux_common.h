@@ -252,12 +252,12 @@ __device__ __forceinline__ void load_rec(const double* rec, int ld, int i, doubl
 
 // left/right states of a face from its two cell-record rows ri, rj (in
 // registers, or ri in LDS): spatial extrapolation + GIZMO, then the
-// half-step predictor
-template <int D>
+// half-step predictor; M: the arithmetic (quot_dev.h)
+template <int D, class M>
 __device__ __forceinline__ void face_states_rows(const double* ri, const double* rj,
                                                  const double* com, double diff, const double* fv,
                                                  double gamma, double dt, int boost, int gizmo,
-                                                 int stages, double* L, double* R)
+                                                 int stages, M& m, double* L, double* R)
 {
     using Y = Lay<D>;
     const double* pi = ri + Y::P0;
@@ -265,20 +265,20 @@ __device__ __forceinline__ void face_states_rows(const double* ri, const double*
     if (stages & PHD_STAGE_SPATIAL) {
         boost_copy<D>(pi, pj, fv, boost, L, R);
         spatial_states<D>(com, diff, ri + Y::C0, rj + Y::C0, pi, pj, ri + Y::G0, rj + Y::G0,
-                          gizmo, L, R);
+                          gizmo, m, L, R);
     }
     if (stages & PHD_STAGE_TEMPORAL) {
-        temporal_side<D>(pi, ri + Y::G0, fv, boost, gamma, dt, L);
-        temporal_side<D>(pj, rj + Y::G0, fv, boost, gamma, dt, R);
+        temporal_side<D>(pi, ri + Y::G0, fv, boost, gamma, dt, m, L);
+        temporal_side<D>(pj, rj + Y::G0, fv, boost, gamma, dt, m, R);
     }
 }
 
 // left/right states of face m into L, R (primitive group, face frame)
-template <int D, int ORDER>
+template <int D, int ORDER, class M>
 __device__ __forceinline__ void face_states(const phd_cells& c, const double* rec, int ld, int i,
                                             int j, const double* com, double diff,
                                             const double* fv, double gamma, double dt, int boost,
-                                            int gizmo, int stages, double* L, double* R)
+                                            int gizmo, int stages, M& m, double* L, double* R)
 {
     using Y = Lay<D>;
     if (ORDER == PHD_ORDER_CONSTANT) {
@@ -291,7 +291,22 @@ __device__ __forceinline__ void face_states(const phd_cells& c, const double* re
     double ri[Y::LD], rj[Y::LD];
     load_rec<D>(rec, ld, i, ri);
     load_rec<D>(rec, ld, j, rj);
-    face_states_rows<D>(ri, rj, com, diff, fv, gamma, dt, boost, gizmo, stages, L, R);
+    face_states_rows<D>(ri, rj, com, diff, fv, gamma, dt, boost, gizmo, stages, m, L, R);
+}
+
+// States and solver of face m in the arithmetic ar, without the deboost; ar.ok
+// says whether F holds (false: an operand left the ranges Shared takes).
+template <int D, int ORDER, int SOLVER, class M>
+__device__ __forceinline__ void face_flux(const phd_cells& c, const double* frec,
+                                          const double* rec, int ld, long long m, int i, int j,
+                                          const double* fv, const Gas& gas, double dt, int boost,
+                                          int gizmo, M& ar, double& area, double* F)
+{
+    double com[D], n[D], diff, L[D + 2], R[D + 2];
+    load_face_rec<D>(frec, m, com, area, n, diff);
+    face_states<D, ORDER>(c, rec, ld, i, j, com, diff, fv, gas.gamma, dt, boost, gizmo,
+                          PHD_STAGE_SPATIAL | PHD_STAGE_TEMPORAL, ar, L, R);
+    riemann_hll<D, SOLVER>(L, R, n, fv, gas, boost, ar, F);
 }
 
 } // namespace

@@ -37,6 +37,7 @@
 // within 2^-20 of one, its binomial series) round differently.
 #include <string.h>
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 #include "flux_common.h"
 
@@ -919,7 +920,8 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_states(phd_cells c, phd_faces f,
 #pragma unroll
         for (int q = 0; q < NF; q++) { L[q] = left.q[q][m]; R[q] = right.q[q][m]; }
     }
-    face_states<D, ORDER>(c, rec, ld, i, j, com, diff, fv, gamma, dt, boost, gizmo, stages, L, R);
+    Ieee ar;
+    face_states<D, ORDER>(c, rec, ld, i, j, com, diff, fv, gamma, dt, boost, gizmo, stages, ar, L, R);
 #pragma unroll
     for (int q = 0; q < NF; q++) { left.q[q][m] = L[q]; right.q[q][m] = R[q]; }
 }
@@ -985,15 +987,39 @@ __global__ __launch_bounds__(BS) void k_face(phd_cells c, phd_faces f,
             return;
         }
     }
-    double com[D], n[D], area, diff, fv[D], L[NF], R[NF], F[NF];
-    load_face_rec<D>(frec, m, com, area, n, diff);
+    double area, fv[D], F[NF];
 #pragma unroll
     for (int k = 0; k < D; k++) fv[k] = BATCH ? 0.0 : f.velocity[k][m];   // batches: static meshes
-    face_states<D, ORDER>(c, rec, ld, i, j, com, diff, fv, gas.gamma, dt_half, boost, gizmo,
-                          PHD_STAGE_SPATIAL | PHD_STAGE_TEMPORAL, L, R);
-    if (!solve_face<D, SOLVER>(L, R, n, fv, gas, boost, F)) {
-        atomicMin(&err[2], (unsigned long long)m);
-        return;
+    if constexpr (SOLVER == PHD_SOLVER_EXACT) {
+        double com[D], n[D], diff, L[NF], R[NF];
+        Ieee ar;
+        load_face_rec<D>(frec, m, com, area, n, diff);
+        face_states<D, ORDER>(c, rec, ld, i, j, com, diff, fv, gas.gamma, dt_half, boost, gizmo,
+                              PHD_STAGE_SPATIAL | PHD_STAGE_TEMPORAL, ar, L, R);
+        if (!solve_face<D, SOLVER>(L, R, n, fv, gas, boost, F)) {
+            atomicMin(&err[2], (unsigned long long)m);
+            return;
+        }
+    } else {
+        // 2D: the quotients and roots are half of the instructions the kernel
+        // is bound by (4096-problem mix, 11.8 M faces: 535 -> 472 us).  3D: it
+        // waits on its record gathers instead (1126 -> 962 VALU instructions a
+        // wave took 128^3 Sedov from 725 to 760 us), and keeps the operators.
+        typename std::conditional<D == 2, Shared, Ieee>::type ar;
+        if (D == 2) ar.ok = gas.shared;
+        face_flux<D, ORDER, SOLVER>(c, frec, rec, ld, m, i, j, fv, gas, dt_half, boost, gizmo, ar,
+                                    area, F);
+        if (D == 2 && !ar.ok) {
+            // rows and record are read again through addresses of their own,
+            // so that nothing is held for this across the first evaluation
+            long long m2 = m;
+            int i2 = i, j2 = j;
+            asm volatile("" : "+v"(m2), "+v"(i2), "+v"(j2));
+            Ieee again;
+            face_flux<D, ORDER, SOLVER>(c, frec, rec, ld, m2, i2, j2, fv, gas, dt_half, boost, gizmo,
+                                        again, area, F);
+        }
+        if (boost) deboost<D>(fv, F);
     }
     if (OUT & 1) {
 #pragma unroll

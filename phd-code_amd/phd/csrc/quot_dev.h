@@ -1,0 +1,125 @@
+// quot_dev.h -- how a face's quotients and square roots are evaluated.
+//
+// The face functions (riemann_dev.h, states_dev.h) take an arithmetic policy:
+//
+//   Ieee    the language's / and sqrt.  Always right.
+//   Shared  the same quotients and roots, bit for bit, for operands whose
+//           ranges have been checked, at a fraction of the instructions.
+//
+// hipcc lowers a / b to two div_scale, rcp, two Newton steps on the
+// reciprocal, q = a r, e = a - b q, div_fmas and div_fixup (11 instructions,
+// 57 cycles a wavefront on MI355X with the quarter-rate rcp), and sqrt to an
+// rsq, a Goldschmidt iteration with two residual corrections, and the scaling
+// of tiny arguments (85 cycles).  Far from the overflow and underflow limits
+// the scaling steps are identities; leaving them out, and computing a
+// divisor's reciprocal once for all its numerators, gives the same correctly
+// rounded results (Markstein 1990: q + e r with q = a r, e = a - b q exact, is
+// the correctly rounded quotient) in 8 instructions per divisor and 3 per
+// numerator, 10 for a root.  A face of the 3D HLLC kernel has about 30
+// quotients and 8 roots, two thirds of its issue slots.
+//
+// Shared keeps one flag: `ok` falls when an operand leaves the ranges for
+// which the comment at the place shows the sequence to be exact, and the
+// caller then evaluates the face again with Ieee.  Every check is written so
+// that a NaN fails it.
+//
+// The residual's form carries the sign of a zero numerator: div() is for
+// divisors > 0, divn() for divisors < 0; the two agree for other numerators.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <math.h>
+
+#ifndef PHD_HD
+#define PHD_HD __host__ __device__
+#endif
+
+namespace phd {
+
+struct Ieee {
+    using Rcp = double;                       // the divisor itself
+    static constexpr bool fast = false;
+    bool ok = true;
+    PHD_HD __forceinline__ Rcp rcp(double b) const { return b; }
+    PHD_HD __forceinline__ Rcp twice(Rcp c) const { return 2. * c; }
+    PHD_HD __forceinline__ Rcp pick(bool first, Rcp a, Rcp b) const { return first ? a : b; }
+    PHD_HD __forceinline__ double div(double a, Rcp c) const { return a / c; }
+    PHD_HD __forceinline__ double divn(double a, Rcp c) const { return a / c; }
+    PHD_HD __forceinline__ double root(double x) const { return sqrt(x); }
+    PHD_HD __forceinline__ void need(bool) {}
+};
+
+// divisor and the reciprocal two Newton steps give
+struct SharedRcp {
+    double b, r;
+};
+
+struct Shared {
+    using Rcp = SharedRcp;
+    static constexpr bool fast = true;
+    bool ok = true;
+
+    // |b| in [2^-310, 2^610]
+    PHD_HD __forceinline__ Rcp rcp(double b) const
+    {
+#ifdef __HIP_DEVICE_COMPILE__
+        double r = __builtin_amdgcn_rcp(b);
+        double e = fma(-b, r, 1.0);
+        r = fma(r, e, r);
+        e = fma(-b, r, 1.0);
+        return {b, fma(r, e, r)};
+#else
+        return {b, 1.0 / b};
+#endif
+    }
+    PHD_HD __forceinline__ Rcp twice(Rcp c) const { return {2. * c.b, .5 * c.r}; }
+    PHD_HD __forceinline__ Rcp pick(bool first, Rcp a, Rcp b) const
+    {
+        return {first ? a.b : b.b, first ? a.r : b.r};
+    }
+    // a zero or |a| in [2^-760, 2^700], |a / b| in [2^-1000, 2^1000] or zero:
+    // the residual is then exact (a multiple of 2^-1074).  A smaller nonzero
+    // a is fine where only 1 + a/b is used.
+    PHD_HD __forceinline__ double div(double a, Rcp c) const
+    {
+        const double q = a * c.r;
+        const double e = fma(c.b, q, -a);
+        return fma(-e, c.r, q);
+    }
+    PHD_HD __forceinline__ double divn(double a, Rcp c) const
+    {
+        const double q = a * c.r;
+        const double e = fma(-c.b, q, a);
+        return fma(e, c.r, q);
+    }
+    // x in [2^-700, 2^1000]
+    PHD_HD __forceinline__ double root(double x) const
+    {
+#ifdef __HIP_DEVICE_COMPILE__
+        const double y = __builtin_amdgcn_rsq(x);
+        double g = x * y, h = y * 0.5;
+        const double r = fma(-h, g, 0.5);
+        g = fma(g, r, g);
+        h = fma(h, r, h);
+        double d = fma(-g, g, x);
+        g = fma(d, h, g);
+        d = fma(-g, g, x);
+        return fma(d, h, g);
+#else
+        return sqrt(x);
+#endif
+    }
+    PHD_HD __forceinline__ void need(bool c) { ok &= c; }
+};
+
+// range checks; all false for NaN
+PHD_HD __forceinline__ bool within(double x, double lo, double hi) { return (x >= lo) & (x <= hi); }
+PHD_HD __forceinline__ bool zero_or_above(double x, double lo)
+{
+    const double a = fabs(x);
+    return (a >= lo) | (x == 0.0);
+}
+// densities and pressures, and the ratios of specific heats, that Shared takes
+PHD_HD __forceinline__ bool state_ok(double x) { return within(x, 0x1p-100, 0x1p100); }
+inline bool shared_gamma(double gamma) { return gamma >= 1. + 0x1p-10 && gamma <= 64.; }
+
+} // namespace phd

@@ -7,6 +7,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "phd_flux.h"
+#include "quot_dev.h"
 
 // callable from kernels and from host code (the host build runs the same
 // functions for the CPU checks of the adjoint)
@@ -26,6 +27,10 @@ struct Gas {
     double inv_z;    // 1./z                            riemann.pyx:460-461
     double gp1_2g;   // (gamma+1.)/(2.*gamma)           riemann.pyx:488,497
     double gm1_gp1;  // (gamma - 1.)/(gamma + 1.)       riemann.pyx:470-471
+    double inv_gm1;  // 1/(gamma - 1.), for quotients by the uniform gamma - 1.
+    bool shared;     // gamma lies where the Shared arithmetic may be used
+    PHD_HD __forceinline__ double gm1(const Ieee&) const { return gamma - 1.; }
+    PHD_HD __forceinline__ SharedRcp gm1(const Shared&) const { return {gamma - 1., inv_gm1}; }
 };
 
 inline Gas make_gas(double gamma)
@@ -36,6 +41,8 @@ inline Gas make_gas(double gamma)
     g.inv_z = 1. / g.z;
     g.gp1_2g = (gamma + 1.) / (2. * gamma);
     g.gm1_gp1 = (gamma - 1.) / (gamma + 1.);
+    g.inv_gm1 = 1. / (gamma - 1.);
+    g.shared = shared_gamma(gamma);
     return g;
 }
 
@@ -58,60 +65,94 @@ PHD_HD __forceinline__ double pow_b1(double x, double y)
 }
 
 // HLL.get_waves (riemann.pyx:375-504): Toro PVRS / TRRS / TSRS p* estimate
-// and Toro eq. 10.68-10.70 wave speeds.
-PHD_HD __forceinline__ void get_waves(double dl, double ul, double pl, double dr, double ur,
-                                          double pr, const Gas& g, double& sl, double& sc,
-                                          double& sr)
+// and Toro eq. 10.68-10.70 wave speeds.  M: the arithmetic (quot_dev.h); rdl,
+// rdr its reciprocals of dl, dr.
+//
+// What Shared's checks give.  d, p in [2^-100, 2^100] and gamma in [1 + 2^-10,
+// 64] put c in [2^-34, 2^104]; |u| zero or in [2^-500, 2^100] bounds p* of the
+// first estimate by 2^310.  TRRS: (pl/pr)^z lies in [2^-100, 2^100], so the
+// numerators of u* are zero or >= 2^-760 and its divisor lies in [2^-205,
+// 2^140]; the two base quotients are only added to 1.  TSRS: every divisor lies
+// in [2^-211, 2^311], p* below 2^430.  The p* that results is checked, which
+// also sends NaN and overflow of the powers to Ieee.  p*/p - 1 is taken only
+// for p* > p, so the roots' arguments are >= 1.  sc: divisor < 0, checked with
+// its numerator.  max/min < 2 rounds to nearest as max < 2 min does for
+// positive p: the quotient of floats below 2 min is at most 2 - 2^-52.
+template <class M>
+PHD_HD __forceinline__ void get_waves_m(double dl, double ul, double pl, double dr, double ur,
+                                        double pr, const Gas& g, M& m, typename M::Rcp rdl,
+                                        typename M::Rcp rdr, double& sl, double& sc, double& sr)
 {
     const double gamma = g.gamma;
     const double Q = 2., c_floor = 1.0E-10;
-    double cl = fmax(sqrt(gamma * pl / dl), c_floor);
-    double cr = fmax(sqrt(gamma * pr / dr), c_floor);
+    m.need(state_ok(dl) & state_ok(pl) & state_ok(dr) & state_ok(pr));
+    m.need(zero_or_above(ul, 0x1p-500) & zero_or_above(ur, 0x1p-500));
+    m.need((fabs(ul) <= 0x1p100) & (fabs(ur) <= 0x1p100));
+    double cl = fmax(m.root(m.div(gamma * pl, rdl)), c_floor);
+    double cr = fmax(m.root(m.div(gamma * pr, rdr)), c_floor);
     double d_avg = .5 * (dl + dr);
     double c_avg = .5 * (cl + cr);
     double p_star = fmax(0., .5 * (pl + pr) + .5 * (ul - ur) * d_avg * c_avg);
     double p_min = fmin(pl, pr);
     double p_max = fmax(pl, pr);
-    if (((p_max / p_min) < Q) && ((p_min < p_star) && (p_star < p_max))) {
+    const bool near = M::fast ? p_max < Q * p_min : (p_max / p_min) < Q;
+    const typename M::Rcp rpr = m.rcp(pr);
+    if (near && ((p_min < p_star) && (p_star < p_max))) {
         // PVRS: p_star kept (u_star at 445 is not used further)
     } else if (p_star <= p_min) {
-        double plr = pow_b1(pl / pr, g.z);
-        double u_star = (plr * ul / cl + ur / cr + 2. * (plr - 1.) / (gamma - 1.)) /
-                        (plr / cl + 1. / cr);
-        p_star = .5 * pl * pow_b1(1. + (gamma - 1.) * (ul - u_star) / (2. * cl), g.inv_z);
-        p_star += .5 * pr * pow_b1(1. + (gamma - 1.) * (u_star - ur) / (2. * cr), g.inv_z);
+        const typename M::Rcp rcl = m.rcp(cl), rcr = m.rcp(cr);
+        double plr = pow_b1(m.div(pl, rpr), g.z);
+        double u_star = m.div(m.div(plr * ul, rcl) + m.div(ur, rcr) + m.div(2. * (plr - 1.), g.gm1(m)),
+                              m.rcp(m.div(plr, rcl) + m.div(1., rcr)));
+        p_star = .5 * pl * pow_b1(1. + m.div((gamma - 1.) * (ul - u_star), m.twice(rcl)), g.inv_z);
+        p_star += .5 * pr * pow_b1(1. + m.div((gamma - 1.) * (u_star - ur), m.twice(rcr)), g.inv_z);
     } else {
-        double Al = 2. / ((gamma + 1.) * dl);
-        double Ar = 2. / ((gamma + 1.) * dr);
+        double Al = m.div(2., m.rcp((gamma + 1.) * dl));
+        double Ar = m.div(2., m.rcp((gamma + 1.) * dr));
         double Bl = pl * g.gm1_gp1;
         double Br = pr * g.gm1_gp1;
-        double gl = sqrt(Al / (p_star + Bl));
-        double gr = sqrt(Ar / (p_star + Br));
-        p_star = (gl * pl + gr * pr - (ur - ul)) / (gl + gr);
+        double gl = m.root(m.div(Al, m.rcp(p_star + Bl)));
+        double gr = m.root(m.div(Ar, m.rcp(p_star + Br)));
+        p_star = m.div(gl * pl + gr * pr - (ur - ul), m.rcp(gl + gr));
     }
+    m.need(p_star <= 0x1p600);
     if (p_star <= pl) sl = ul - cl;
-    else sl = ul - cl * sqrt(1. + g.gp1_2g * (p_star / pl - 1.));
+    else sl = ul - cl * m.root(1. + g.gp1_2g * (m.div(p_star, m.rcp(pl)) - 1.));
     if (p_star <= pr) sr = ur + cr;
-    else sr = ur + cr * sqrt(1. + g.gp1_2g * (p_star / pr - 1.));
-    sc = (pr - pl + dl * ul * (sl - ul) - dr * ur * (sr - ur)) / (dl * (sl - ul) - dr * (sr - ur));
+    else sr = ur + cr * m.root(1. + g.gp1_2g * (m.div(p_star, rpr) - 1.));
+    const double num = pr - pl + dl * ul * (sl - ul) - dr * ur * (sr - ur);
+    const double den = dl * (sl - ul) - dr * (sr - ur);
+    m.need(within(den, -0x1p300, -0x1p-300) & zero_or_above(num, 0x1p-600));
+    sc = m.divn(num, m.rcp(den));
+}
+
+PHD_HD __forceinline__ void get_waves(double dl, double ul, double pl, double dr, double ur,
+                                      double pr, const Gas& g, double& sl, double& sc, double& sr)
+{
+    Ieee m;
+    get_waves_m(dl, ul, pl, dr, ur, pr, g, m, dl, dr, sl, sc, sr);
 }
 
 // pure upwind state flux in the moving frame (riemann.pyx:624-631, 672-679)
-template <int D>
+template <int D, class M>
 PHD_HD __forceinline__ void side_flux(const double* S, const double* n, double Vn, double vsq,
-                                          double wn, double gamma, double* F)
+                                          double wn, const Gas& g, M& m, double* F)
 {
     double d = S[0], p = S[D + 1];
     F[0] = d * (Vn - wn);
-    F[D + 1] = (0.5 * d * vsq + p / (gamma - 1.0)) * (Vn - wn) + p * Vn;
+    F[D + 1] = (0.5 * d * vsq + m.div(p, g.gm1(m))) * (Vn - wn) + p * Vn;
 #pragma unroll
     for (int k = 0; k < D; k++) F[1 + k] = d * S[1 + k] * (Vn - wn) + p * n[k];
 }
 
-// HLL (riemann.pyx:243-373) and HLLC (riemann.pyx:521-682) interface flux
-template <int D, int SOLVER>
+// HLL (riemann.pyx:243-373) and HLLC (riemann.pyx:521-682) interface flux.
+// Shared: the star flux's mass flux into the wave d (s - Vn), which is a
+// numerator and part of a divisor, and s - sc are checked nonzero and in
+// range, so the signs of their quotients' zeros play no part; e >= p/(gamma-1).
+template <int D, int SOLVER, class M>
 PHD_HD __forceinline__ void riemann_hll(const double* L, const double* R, const double* n,
-                                            const double* fv, const Gas& g, int boost, double* F)
+                                            const double* fv, const Gas& g, int boost, M& m,
+                                            double* F)
 {
     const double gamma = g.gamma;
     double _dl = L[0], _pl = L[D + 1], _dr = R[0], _pr = R[D + 1];
@@ -126,7 +167,8 @@ PHD_HD __forceinline__ void riemann_hll(const double* L, const double* R, const 
     }
     if (boost) wn = 0.;
     double sl, sc, sr;
-    get_waves(_dl, Vnl, _pl, _dr, Vnr, _pr, g, sl, sc, sr);
+    const typename M::Rcp rdl = m.rcp(_dl), rdr = m.rcp(_dr);
+    get_waves_m(_dl, Vnl, _pl, _dr, Vnr, _pr, g, m, rdl, rdr, sl, sc, sr);
     if (SOLVER == PHD_SOLVER_HLL && (sl < wn) && (wn <= sr)) {
         // Toro eq. 10.20-10.21 (riemann.pyx:346-361)
         double fac1 = sr - wn, fac2 = sl - wn, fac3 = sr - sl;
@@ -155,19 +197,31 @@ PHD_HD __forceinline__ void riemann_hll(const double* L, const double* R, const 
         const double d = S[0], p = S[D + 1];
         const double Vn = left ? Vnl : Vnr, vsq = left ? vl_sq : vr_sq, s = left ? sl : sr;
         if (SOLVER == PHD_SOLVER_HLLC && mid) {
-            double factor_1 = d * (s - Vn) / (s - sc);
+            const double into = d * (s - Vn), gap = s - sc;
+            m.need(within(fabs(into), 0x1p-300, 0x1p300) & within(fabs(gap), 0x1p-300, 0x1p300));
+            double factor_1 = m.div(into, m.rcp(gap));
             double factor_2 = factor_1 * (s - wn) * (sc - Vn) + p;
             double frho = d * (Vn - s) + factor_1 * (s - wn);
-            double e = 0.5 * d * vsq + p / (gamma - 1.0);
+            double e = 0.5 * d * vsq + m.div(p, g.gm1(m));
+            m.need(e <= 0x1p600);
             F[0] = frho;
             F[D + 1] = (e + p) * Vn - s * e +
-                       (s - wn) * factor_1 * (e / d + (sc - Vn) * (sc + p / (d * (s - Vn))));
+                       (s - wn) * factor_1 * (m.div(e, m.pick(left, rdl, rdr)) +
+                                              (sc - Vn) * (sc + m.div(p, m.rcp(into))));
 #pragma unroll
             for (int k = 0; k < D; k++) F[1 + k] = frho * S[1 + k] + factor_2 * n[k];
         } else {
-            side_flux<D>(S, n, Vn, vsq, wn, gamma, F);
+            side_flux<D>(S, n, Vn, vsq, wn, g, m, F);
         }
     }
+}
+
+template <int D, int SOLVER>
+PHD_HD __forceinline__ void riemann_hll(const double* L, const double* R, const double* n,
+                                            const double* fv, const Gas& g, int boost, double* F)
+{
+    Ieee m;
+    riemann_hll<D, SOLVER>(L, R, n, fv, g, boost, m, F);
 }
 
 // RiemannBase.deboost (riemann.pyx:190-222), Pakmor & Springel (2011) eq. 17

@@ -1,0 +1,58 @@
+// Host build of the face functions under both arithmetics of quot_dev.h, for
+// tests/test_quotients_cpu.py.  Test infrastructure: nothing in the library
+// loads it.
+#include <hip/hip_runtime.h>
+#include <string.h>
+#include "riemann_dev.h"
+#include "states_dev.h"
+
+using namespace phd;
+
+namespace {
+
+template <int D, int SOLVER, class M>
+bool face(const double* ri, const double* rj, const double* com, double diff, const double* n,
+          const double* fv, const Gas& g, double dt, int boost, int gizmo, M& m, double* F)
+{
+    constexpr int NF = D + 2, G0 = NF, C0 = NF + D * NF;
+    double L[NF], R[NF];
+    boost_copy<D>(ri, rj, fv, boost, L, R);
+    spatial_states<D>(com, diff, ri + C0, rj + C0, ri, rj, ri + G0, rj + G0, gizmo, m, L, R);
+    temporal_side<D>(ri, ri + G0, fv, boost, g.gamma, dt, m, L);
+    temporal_side<D>(rj, rj + G0, fv, boost, g.gamma, dt, m, R);
+    riemann_hll<D, SOLVER>(L, R, n, fv, g, boost, m, F);
+    return m.ok;
+}
+
+template <int D, int SOLVER>
+void faces(long nf, const double* ri, const double* rj, const double* com, const double* diff,
+           const double* n, const double* fv, double gamma, double dt, int boost, int gizmo,
+           unsigned char* ok, unsigned char* same)
+{
+    constexpr int NF = D + 2, W = NF + D * NF + D;
+    const Gas g = make_gas(gamma);
+    for (long f = 0; f < nf; f++) {
+        double A[NF], B[NF];
+        Ieee mi;
+        Shared ms;
+        ms.ok = g.shared;
+        face<D, SOLVER>(ri + f * W, rj + f * W, com + f * D, diff[f], n + f * D, fv + f * D, g, dt,
+                        boost, gizmo, mi, A);
+        ok[f] = face<D, SOLVER>(ri + f * W, rj + f * W, com + f * D, diff[f], n + f * D, fv + f * D,
+                                g, dt, boost, gizmo, ms, B);
+        same[f] = memcmp(A, B, sizeof(A)) == 0;
+    }
+}
+
+} // namespace
+
+extern "C" void qh_faces(int dim, int hllc, long nf, const double* ri, const double* rj,
+                         const double* com, const double* diff, const double* n, const double* fv,
+                         double gamma, double dt, int boost, int gizmo, unsigned char* ok,
+                         unsigned char* same)
+{
+    if (dim == 2 && hllc) faces<2, PHD_SOLVER_HLLC>(nf, ri, rj, com, diff, n, fv, gamma, dt, boost, gizmo, ok, same);
+    else if (dim == 2) faces<2, PHD_SOLVER_HLL>(nf, ri, rj, com, diff, n, fv, gamma, dt, boost, gizmo, ok, same);
+    else if (hllc) faces<3, PHD_SOLVER_HLLC>(nf, ri, rj, com, diff, n, fv, gamma, dt, boost, gizmo, ok, same);
+    else faces<3, PHD_SOLVER_HLL>(nf, ri, rj, com, diff, n, fv, gamma, dt, boost, gizmo, ok, same);
+}
