@@ -103,21 +103,29 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_prim_from_cons(phd_cells c, doubl
     c.prim[D + 1][i] = (c.cons[D + 1][i] / vol - .5 * d * v_sq) * (gamma - 1.);
 }
 
+// CFL minimum of all real cells into err[3].  Every block ends with one atomic
+// minimum on the same word, about 12 ns each whatever the chip does meanwhile:
+// one per 256 cells took 102 us at 128^3 (the 53 MB read take 9).  So at most
+// CFL_BLOCKS blocks of 1024 threads, one a CU, walk the cells: 27 us there (the
+// pow of each cell's radius bounds it now), and 14.8 -> 6.9 us at 512^2 in 2D.
+constexpr int CFL_THREADS = 1024, CFL_BLOCKS = 256;
+
 template <int D>
-__global__ __launch_bounds__(PHD_BLOCK) void k_cfl(phd_cells c, double gamma, int boost,
-                                                   unsigned long long* err)
+__global__ __launch_bounds__(CFL_THREADS) void k_cfl(phd_cells c, double gamma, int boost,
+                                                     unsigned long long* err)
 {
-    long long i = (long long)blockIdx.x * PHD_BLOCK + threadIdx.x;
     double v = __longlong_as_double((long long)INF_BITS);
-    if (i < c.n_cells && c.tag[i] == 0) v = cfl_value<D>(c, i, gamma, boost);
+    for (long long i = (long long)blockIdx.x * CFL_THREADS + threadIdx.x; i < c.n_cells;
+         i += (long long)gridDim.x * CFL_THREADS)
+        if (c.tag[i] == 0) v = fmin(v, cfl_value<D>(c, i, gamma, boost));
     for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-    __shared__ double wmin[PHD_BLOCK / 64];
+    __shared__ double wmin[CFL_THREADS / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0) wmin[wid] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         double b = wmin[0];
-        for (int w = 1; w < PHD_BLOCK / 64; w++) b = fmin(b, wmin[w]);
+        for (int w = 1; w < CFL_THREADS / 64; w++) b = fmin(b, wmin[w]);
         atomicMin(&err[3], (unsigned long long)__double_as_longlong(b));
     }
 }
@@ -2002,8 +2010,9 @@ int phd_compute_time_step(phd_handle* h, const phd_cells* c, double gamma, doubl
     if (!h || check_cells(c) || !dt_out || c->n_cells == 0) return PHD_E_ARG;
     k_reset_err<<<1, 64, 0, h->stream>>>(h->d_err);   // also clears the fault words
     LAUNCHCHK();
-    if (c->dim == 2) k_cfl<2><<<nblocks(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, gamma, boost, h->d_err);
-    else k_cfl<3><<<nblocks(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, gamma, boost, h->d_err);
+    const int nb = std::min((c->n_cells - 1) / CFL_THREADS + 1, CFL_BLOCKS);
+    if (c->dim == 2) k_cfl<2><<<nb, CFL_THREADS, 0, h->stream>>>(*c, gamma, boost, h->d_err);
+    else k_cfl<3><<<nb, CFL_THREADS, 0, h->stream>>>(*c, gamma, boost, h->d_err);
     LAUNCHCHK();
     HIPCHK(hipMemcpyAsync(h->h_err + 3, h->d_err + 3, sizeof(unsigned long long), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
