@@ -1106,49 +1106,40 @@ __device__ __forceinline__ bool apply_summand(double* u, const double* t, bool i
     return false;
 }
 
-// API path: riemann.fluxes + face areas, per-cell lists from the CSR
-template <int D>
-__global__ __launch_bounds__(PHD_BLOCK) void k_update(phd_cells c, const double* __restrict__ area,
-                                                      FaceArrays flux,
-                                                      const int2* __restrict__ csr,
-                                                      const int32_t* __restrict__ off, double dt,
-                                                      unsigned long long* err)
-{
-    constexpr int NF = D + 2;
-    long long ii = xcd_index(c.n_cells);
-    if (ii >= c.n_cells) return;
-    const int i = (int)ii;
-    const int beg = off[i], end = off[i + 1];
-    if (ghost_fault<D>(c, i, beg, end, csr, err)) return;
-    double u[NF];
-#pragma unroll
-    for (int q = 0; q < NF; q++) u[q] = c.cons[q][i];
-    for (int e = beg; e < end; e++) {
-        const int2 en = csr[e];
-        if ((en.y & 0x7fffffff) == INVALID) continue;
-        const int fid = en.x;
-        double t[NF];
-        const double s = dt * area[fid];
-#pragma unroll
-        for (int q = 0; q < NF; q++) t[q] = s * flux.q[q][fid];
-        if (apply_summand<D>(u, t, en.y & INCOMING, fid, err)) break;
+// Where the update takes a face's summand (dt*area)*flux from: the rows the
+// fused face kernel wrote, or the caller's flux arrays and areas (each product
+// formed as the reference does, mesh.pyx:530-544).
+struct RowSummands {
+    const double* g;
+    template <int D> __device__ __forceinline__ void get(int fid, double* s) const
+    {
+        load_summand<D>(g, fid, s);
     }
-#pragma unroll
-    for (int q = 0; q < NF; q++) c.cons[q][i] = u[q];
-}
+};
 
-// fused-step path: the per-face summand rows g of the face kernel, the
-// per-cell lists as sliced face ids (sfi, coalesced) in the plan's visiting
-// order.  Faces are numbered in owner order, so a cell's list is its
+struct FluxSummands {
+    FaceArrays flux;
+    const double* area;
+    double dt;
+    template <int D> __device__ __forceinline__ void get(int fid, double* s) const
+    {
+        const double t = dt * area[fid];
+#pragma unroll
+        for (int q = 0; q < D + 2; q++) s[q] = t * flux.q[q][fid];
+    }
+};
+
+// The per-cell lists are the sliced face ids (sfi, coalesced) in the plan's
+// visiting order.  Faces are numbered in owner order, so a cell's list is its
 // incoming faces followed by one run of consecutive owned face ids
 // (owner_runs): the incoming rows are gathered, the owned run is read as
 // consecutive rows without touching the list again.
 // Conserved update of the cell at sliced position t (cell i = perm[t]):
 // u = its conserved values plus its summand rows in list order.  False for a
 // ghost (nothing to write; a ghost with faces reports a fault).
-template <int D, int OR>
+template <int D, int OR, class SRC>
 __device__ __forceinline__ bool update_cell(const phd_cells& c, long long t, int i,
-                                            const double* __restrict__ g,
+                                            const SRC& src,
                                             const int2* __restrict__ csr,
                                             const int32_t* __restrict__ off,
                                             const int32_t* __restrict__ sbase,
@@ -1183,7 +1174,7 @@ __device__ __forceinline__ bool update_cell(const phd_cells& c, long long t, int
                             : -1;
 #pragma unroll
             for (int b = 0; b < B; b++)
-                if (fb[b] >= 0) load_summand<D>(g, fb[b], sb[b]);
+                if (fb[b] >= 0) src.template get<D>(fb[b], sb[b]);
 #pragma unroll
             for (int b = 0; b < B; b++)
                 if (!stop && fb[b] >= 0) stop = apply_summand<D>(u, sb[b], true, fb[b], err);
@@ -1192,7 +1183,7 @@ __device__ __forceinline__ bool update_cell(const phd_cells& c, long long t, int
             double sb[B][GW];
 #pragma unroll
             for (int b = 0; b < B; b++)
-                if (k0 + b < n_own) load_summand<D>(g, ci.y + k0 + b, sb[b]);
+                if (k0 + b < n_own) src.template get<D>(ci.y + k0 + b, sb[b]);
 #pragma unroll
             for (int b = 0; b < B; b++)
                 if (!stop && k0 + b < n_own) stop = apply_summand<D>(u, sb[b], false, ci.y + k0 + b, err);
@@ -1203,25 +1194,22 @@ __device__ __forceinline__ bool update_cell(const phd_cells& c, long long t, int
             if (en == INVALID) continue;
             const int fid = en & 0x7fffffff;
             double s[GW];
-            load_summand<D>(g, fid, s);
+            src.template get<D>(fid, s);
             if (apply_summand<D>(u, s, en & INCOMING, fid, err)) break;
         }
     }
     return true;
 }
 
-// OR: the plan's owner_runs flag as a template constant (the kernel holds
-// only the path it takes)
-template <int D, int BS = PHD_BLOCK, int XCD = 1, int OR = 1>
-__global__ __launch_bounds__(BS) void k_update_sell(phd_cells c,
-                                                           const double* __restrict__ g,
-                                                           const int2* __restrict__ csr,
-                                                           const int32_t* __restrict__ off,
-                                                           const int32_t* __restrict__ perm,
-                                                           const int32_t* __restrict__ sbase,
-                                                           const int32_t* __restrict__ sfi,
-                                                           const int2* __restrict__ cinfo,
-                                                           unsigned long long* err)
+template <int D, int BS, int XCD, int OR, class SRC>
+__device__ __forceinline__ void update_body(const phd_cells& c, const SRC& src,
+                                            const int2* __restrict__ csr,
+                                            const int32_t* __restrict__ off,
+                                            const int32_t* __restrict__ perm,
+                                            const int32_t* __restrict__ sbase,
+                                            const int32_t* __restrict__ sfi,
+                                            const int2* __restrict__ cinfo,
+                                            unsigned long long* err)
 {
     // At SORT_WINDOW threads a block owns one whole window (the degree sort
     // permutes within windows): the updated values pass through LDS and are
@@ -1234,7 +1222,7 @@ __global__ __launch_bounds__(BS) void k_update_sell(phd_cells c,
     const long long w0 = t - threadIdx.x;          // the window's first cell
     const int i = t < n ? perm[t] : 0;
     double u[NF];
-    const bool real = t < n && update_cell<D, OR>(c, t, i, g, csr, off, sbase, sfi, cinfo, err, u);
+    const bool real = t < n && update_cell<D, OR>(c, t, i, src, csr, off, sbase, sfi, cinfo, err, u);
     if (!STAGE) {
         if (real) {
 #pragma unroll
@@ -1251,6 +1239,83 @@ __global__ __launch_bounds__(BS) void k_update_sell(phd_cells c,
     if (k < n && c.tag[k] == 0) {
 #pragma unroll
         for (int q = 0; q < NF; q++) c.cons[q][k] = su[q * SORT_WINDOW + threadIdx.x];
+    }
+}
+
+// OR: the plan's owner_runs flag as a template constant (the kernel holds
+// only the path it takes)
+template <int D, int BS = PHD_BLOCK, int XCD = 1, int OR = 1>
+__global__ __launch_bounds__(BS) void k_update_sell(phd_cells c, const double* __restrict__ g,
+                                                    const int2* __restrict__ csr,
+                                                    const int32_t* __restrict__ off,
+                                                    const int32_t* __restrict__ perm,
+                                                    const int32_t* __restrict__ sbase,
+                                                    const int32_t* __restrict__ sfi,
+                                                    const int2* __restrict__ cinfo,
+                                                    unsigned long long* err)
+{
+    update_body<D, BS, XCD, OR>(c, RowSummands{g}, csr, off, perm, sbase, sfi, cinfo, err);
+}
+
+// The update from the caller's flux arrays and areas.  A face gathered from them
+// costs D + 3 cache lines, so the block first forms the summands of its
+// window's owned faces (one id range when the faces are in owner order) in LDS,
+// from coalesced loads, and both cells' entries read them there; the rest are
+// gathered.  CAP rows leave two blocks a CU their LDS in 3D (about 2020 faces a
+// window) and five in 2D (768).  Against a walk of the CSR entries one by one:
+// 512^2 in 2D 41 -> 28 us, 41^3 54 -> 39 us.
+template <int D> constexpr int flux_cap() { return D == 2 ? 800 : 1750; }
+
+struct StagedSummands {
+    FluxSummands far;
+    const double* rows;
+    int f0, n;
+    template <int D> __device__ __forceinline__ void get(int fid, double* s) const
+    {
+        const unsigned k = (unsigned)(fid - f0);
+        if (k < (unsigned)n) {
+#pragma unroll
+            for (int q = 0; q < D + 2; q++) s[q] = rows[k * (D + 2) + q];
+        } else {
+            far.get<D>(fid, s);
+        }
+    }
+};
+
+template <int D, int OR>
+__global__ __launch_bounds__(PHD_BLOCK) void k_update_flux(phd_cells c, int n_faces,
+                                                           FluxSummands src,
+                                                           const int2* __restrict__ csr,
+                                                           const int32_t* __restrict__ off,
+                                                           const int32_t* __restrict__ perm,
+                                                           const int32_t* __restrict__ sbase,
+                                                           const int32_t* __restrict__ sfi,
+                                                           const int2* __restrict__ cinfo,
+                                                           unsigned long long* err)
+{
+    if constexpr (OR) {
+        __shared__ double rows[flux_cap<D>() * (D + 2)];
+        __shared__ int first;
+        const long long t = xcd_index(c.n_cells);
+        if (threadIdx.x == 0) first = n_faces;
+        __syncthreads();
+        if (t < c.n_cells && c.tag[perm[t]] == 0) {
+            const int own0 = cinfo[t].y;           // -1: no owned face
+            if (own0 >= 0) atomicMin(&first, own0);
+        }
+        __syncthreads();
+        const int f0 = first, n = min(flux_cap<D>(), n_faces - f0);
+        for (int k = threadIdx.x; k < n; k += PHD_BLOCK) {
+            double s[D + 2];
+            src.get<D>(f0 + k, s);
+#pragma unroll
+            for (int q = 0; q < D + 2; q++) rows[k * (D + 2) + q] = s[q];
+        }
+        __syncthreads();
+        update_body<D, PHD_BLOCK, 1, OR>(c, StagedSummands{src, rows, f0, n}, csr, off, perm, sbase,
+                                         sfi, cinfo, err);
+    } else {
+        update_body<D, PHD_BLOCK, 1, OR>(c, src, csr, off, perm, sbase, sfi, cinfo, err);
     }
 }
 
@@ -1476,7 +1541,7 @@ __global__ __launch_bounds__(BS) void k_update_eos(phd_cells c, const double* __
     if (threadIdx.x == 0) s_p0 = ws < n ? problem_of((int)ws, bcs, n_problems) : 0;
     double u[NF], p[NF];
     int i = t < n ? perm[t] : 0;
-    bool real = t < n && update_cell<D, OR>(c, t, i, g, csr, off, sbase, sfi, cinfo, err, u);
+    bool real = t < n && update_cell<D, OR>(c, t, i, RowSummands{g}, csr, off, sbase, sfi, cinfo, err, u);
     if (STAGE) {
         if (real) {
 #pragma unroll
@@ -1689,20 +1754,26 @@ int launch_face(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces*
     return PHD_E_MODE;
 }
 
-template <int D, int SRC>
-int launch_update(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces* f,
-                  FaceArrays flux, double dt)
+template <int D>
+int launch_update(phd_handle* h, phd_plan* p, const phd_cells* c)
 {
     if (c->n_cells == 0) return 0;
-    if (SRC == 1 && p->owner_runs)
-        k_update_sell<D, PHD_BLOCK, 1, 1><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(
-            *c, p->g, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err);
-    else if (SRC == 1)
-        k_update_sell<D, PHD_BLOCK, 1, 0><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(
-            *c, p->g, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err);
-    else
-        k_update<D><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(
-            *c, f ? f->area : nullptr, flux, p->csr, p->off, dt, h->d_err);
+#define US(OR) k_update_sell<D, PHD_BLOCK, 1, OR><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, p->g, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
+    if (p->owner_runs) US(1);
+    else US(0);
+#undef US
+    LAUNCHCHK();
+    return 0;
+}
+
+template <int D>
+int launch_update_flux(phd_handle* h, phd_plan* p, const phd_cells* c, const FluxSummands& src)
+{
+    if (c->n_cells == 0) return 0;
+#define UF(OR) k_update_flux<D, OR><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, p->n_faces, src, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
+    if (p->owner_runs) UF(1);
+    else UF(0);
+#undef UF
     LAUNCHCHK();
     return 0;
 }
@@ -2163,9 +2234,8 @@ int phd_update_from_fluxes(phd_handle* h, phd_plan* p, const phd_cells* c, const
     if (!h || check_cells(c) || check_faces(f) || check_plan(p, c) || check_plan_faces(p, f) ||
         !flux)
         return PHD_E_ARG;
-    FaceArrays F = fa(flux, c->dim + 2);
-    return c->dim == 2 ? launch_update<2, 0>(h, p, c, f, F, dt)
-                       : launch_update<3, 0>(h, p, c, f, F, dt);
+    const FluxSummands src{fa(flux, c->dim + 2), f->area, dt};
+    return c->dim == 2 ? launch_update_flux<2>(h, p, c, src) : launch_update_flux<3>(h, p, c, src);
 }
 
 // ---- core-step stages -------------------------------------------------------
@@ -2196,9 +2266,7 @@ int phd_face_summands(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_
 int phd_update_from_summands(phd_handle* h, phd_plan* p, const phd_cells* c)
 {
     if (!h || check_cells(c) || check_plan(p, c)) return PHD_E_ARG;
-    FaceArrays F = fa(nullptr, 0);
-    return c->dim == 2 ? launch_update<2, 1>(h, p, c, nullptr, F, 0.0)
-                       : launch_update<3, 1>(h, p, c, nullptr, F, 0.0);
+    return c->dim == 2 ? launch_update<2>(h, p, c) : launch_update<3>(h, p, c);
 }
 
 // ---- fused core step -----------------------------------------------------------
