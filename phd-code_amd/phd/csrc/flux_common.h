@@ -53,6 +53,7 @@ struct phd_plan {
     int2* cinfo;                 // per position: incoming count, first owned face
     double* sgeo[4];             // face centroid x, y, z, area per slot
     double* g;                   // per-face update summand rows (dt*area)*flux, F x GW
+    int faces_ok;                // every face centroid and area is zero or in [2^-100, 2^100]
     int owner_runs;              // every real cell's owned faces are one id run that
                                  // follows all its incoming faces (faces in owner order)
     int32_t* ghosts;             // third allocation: the ghost cells (tag 1), ascending
@@ -83,7 +84,7 @@ constexpr uint16_t LOC_GLOBAL = 0xFFFE, LOC_NONE = 0xFFFF;   // sloc markers
 // 3D (53 KB of LDS per block, three blocks per CU as its registers allow);
 // none in 2D, where a tenth of the entries lie outside the window and the
 // staging code would cost the kernel its fourth wave per SIMD
-template <int D> constexpr int halo_max() { return D == 2 ? 0 : 576; }
+template <int D> constexpr int halo_max() { return D == 2 ? 112 : 576; }
 
 // Face record: com(D) | area | normal(D) | |x_j - x_i|, 6 doubles in 2D and
 // 8 in 3D (rows stay 16-byte aligned for the paired loads)

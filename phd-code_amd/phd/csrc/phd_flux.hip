@@ -184,8 +184,18 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_face_vel(phd_cells c, phd_faces f
 
 // ---------------------------------------------------------------------------
 // plan construction (once per frozen mesh)
+
+// x == 0 or |x| in [2^-100, 2^100]; false for inf and NaN (non-short-circuit
+// operators: the test compiles to compares and mask logic, no branches)
+__device__ __forceinline__ bool operand_ok(double x)
+{
+    const double ax = fabs(x);
+    return (ax <= 0x1p100) & ((ax >= 0x1p-100) | (x == 0.0));
+}
+
 template <int D>
-__global__ __launch_bounds__(PHD_BLOCK) void k_plan_faces(phd_cells c, phd_faces f, double* rec)
+__global__ __launch_bounds__(PHD_BLOCK) void k_plan_faces(phd_cells c, phd_faces f, double* rec,
+                                                          unsigned long long* flag)
 {
     long long m = xcd_index(f.n_faces);
     if (m >= f.n_faces) return;
@@ -201,6 +211,10 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_plan_faces(phd_cells c, phd_faces
         diff += dx * dx;          // reconstruction.pyx:866
     }
     r[F::A] = f.area[m];
+    bool ok = operand_ok(r[F::A]);
+#pragma unroll
+    for (int k = 0; k < D; k++) ok &= operand_ok(r[F::C + k]);
+    if (!ok) atomicMin(flag, 0ull);
     r[F::DIFF] = sqrt(diff);      // reconstruction.pyx:875
     double2* o = reinterpret_cast<double2*>(rec + (size_t)m * F::W);
 #pragma unroll
@@ -500,39 +514,24 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_pack_xp(phd_cells c, double* xp)
 }
 
 // ---------------------------------------------------------------------------
-// Division by one divisor shared by many numerators.  hipcc lowers a / b on
-// gfx950 to div_scale, rcp, two Newton steps on the reciprocal, q0 = a*r,
-// e = fma(-b, q0, a), div_fmas, div_fixup.  For |a|, |b| in [2^-200, 2^200]
-// div_scale returns its operand unchanged with VCC clear (no operand or
-// quotient is near the overflow/underflow limits), div_fmas reduces to
-// fma(e, r, q0) and div_fixup to the identity, so the steps below give the
-// bits of a / b while the reciprocal and its two Newton steps are computed
-// once per divisor.  The residual is formed as b*q0 - a and subtracted, which
-// is the same exact value with the opposite sign; for b > 0 that makes a zero
-// numerator come out as the correctly signed zero.  Callers check the range
-// and b > 0 and use the ordinary division otherwise.
-__device__ __forceinline__ double rcp_newton(double b)
+// Ranges of the gradient sums' operands, for the Shared arithmetic (quot_dev.h).
+// With every position, primitive, face centroid and area zero or in [2^-100,
+// 2^100] and volumes in [2^-200, 2^100]: differences and sums of them are zero
+// or >= 2^-153, the distance r = sqrt(sum dr^2) lies in [2^-153, 2^102] unless
+// zero, r * vol in [2^-353, 2^202], and the numerators area * (...) are zero or
+// in [2^-459, 2^304].  So the values are checked once, where a row is staged and
+// (the faces) where the plan is made, and not the numerators of every entry.
+//
+// row_ok: every value of a packed row that the gradients take
+template <int D>
+__device__ __forceinline__ bool row_ok(const double* r)
 {
-    double r = __builtin_amdgcn_rcp(b);
-    double e = fma(-b, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-b, r, 1.0);
-    return fma(r, e, r);
-}
-
-__device__ __forceinline__ double div_shared(double a, double b, double r)
-{
-    const double q = a * r;
-    const double e = fma(b, q, -a);
-    return fma(-e, r, q);
-}
-
-// |x| in [2^-200, 2^200] or x == 0; false for inf and NaN (non-short-circuit
-// operators: the test compiles to compares and mask logic, no branches)
-__device__ __forceinline__ bool div_operand_ok(double x)
-{
-    const double ax = fabs(x);
-    return (ax <= 0x1p200) & ((ax >= 0x1p-200) | (x == 0.0));
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < D; k++) ok &= operand_ok(r[XpLay<D>::X + k]);
+#pragma unroll
+    for (int n = 0; n < D + 2; n++) ok &= operand_ok(r[XpLay<D>::P + n]);
+    return ok;
 }
 
 // one entry of a sliced list: neighbour id (INCOMING bit cleared), face
@@ -577,8 +576,11 @@ __device__ __forceinline__ void load_row(const double* xp, int j, double* r)
 // correctly rounded quotient is monotone in its divisor, so the minimum over
 // faces is reached at the largest positive dphi and at the most negative
 // dphi: two divisions per field instead of one per face, same bits.
+//
+// Registers: 2D is held to 128 (4 waves per SIMD, no spills; it would take 129).
 template <int D, int LIM, int BS = PHD_BLOCK, int XCD = 1>
-__global__ __launch_bounds__(BS) void k_grad_sell(int n_cells, const int8_t* __restrict__ tag,
+__global__ __launch_bounds__(BS)
+__attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cells, const int8_t* __restrict__ tag,
                                                          const double* __restrict__ geo,
                                                          const double* __restrict__ vols,
                                                          const double* __restrict__ xp,
@@ -593,6 +595,7 @@ __global__ __launch_bounds__(BS) void k_grad_sell(int n_cells, const int8_t* __r
                                                          const int32_t* __restrict__ hcnt,
                                                          const int32_t* __restrict__ halo,
                                                          const uint16_t* __restrict__ sloc,
+                                                         int faces_ok,
                                                          double* __restrict__ rec, int ld)
 {
     using Y = Lay<D>;
@@ -608,7 +611,6 @@ __global__ __launch_bounds__(BS) void k_grad_sell(int n_cells, const int8_t* __r
     constexpr bool STAGE = BS == SORT_WINDOW;
     constexpr int HM = STAGE ? halo_max<D>() : 0;
     constexpr bool HALO = HM > 0;
-    __shared__ double2 rows[STAGE ? (SORT_WINDOW + HM) * XPW / 2 : 1];
     // 2D AREPO: the first KC entries of each list keep their face centroid
     // in LDS from the gradient pass for the limiter pass ([entry][thread],
     // thread-private), so the limiter streams only the later slots again.
@@ -616,7 +618,18 @@ __global__ __launch_bounds__(BS) void k_grad_sell(int n_cells, const int8_t* __r
     // allow (4096-problem step -0.8 %).  In 3D the 6 entries that would fit
     // beside three blocks changed nothing measurable.
     constexpr int KC = STAGE && LIM == PHD_LIMITER_AREPO && D == 2 ? 4 : 0;
-    __shared__ double2 ccache[KC > 0 ? KC * SORT_WINDOW : 1];
+    // 2D: the block's records leave through the same LDS, in natural order as
+    // one stream (a lane storing its own record touches a line per 16 bytes:
+    // 421 -> 367 us on the 256-problem ensemble).  In 3D the values held past
+    // the barrier cost a wave per SIMD or spill (573 us, 688 or 579).
+    constexpr bool STREAM = STAGE && D == 2;
+    constexpr int Q = Y::LD / 2;
+    constexpr int NROWS = (SORT_WINDOW + HM) * XPW / 2, NCACHE = KC * SORT_WINDOW;
+    constexpr int NOUT = STREAM ? SORT_WINDOW * Q : 0;
+    __shared__ double2 lds[STAGE ? (NROWS + NCACHE > NOUT ? NROWS + NCACHE : NOUT) : 1];
+    __shared__ unsigned char written[STREAM ? SORT_WINDOW : 1];
+    double2* const rows = lds;
+    double2* const ccache = lds + NROWS;
     const long long t = sched_index<BS, XCD>(n_cells);
     const bool live = t < n_cells;
     const int i = live ? perm[t] : 0;
@@ -626,8 +639,10 @@ __global__ __launch_bounds__(BS) void k_grad_sell(int n_cells, const int8_t* __r
 #pragma unroll
         for (int q = 0; q < XPW / 2; q++) ld2(xp + (size_t)i * XPW + 2 * q, own[2 * q], own[2 * q + 1]);
     }
+    bool fast = faces_ok != 0;
     if (STAGE) {
         if (live) {
+            fast &= row_ok<D>(own);
 #pragma unroll
             for (int q = 0; q < XPW / 2; q++)
                 rows[(i - w0) * (XPW / 2) + q] = make_double2(own[2 * q], own[2 * q + 1]);
@@ -636,252 +651,263 @@ __global__ __launch_bounds__(BS) void k_grad_sell(int n_cells, const int8_t* __r
             const long long w = w0 / SORT_WINDOW;
             const int hn = hcnt[w];                // at most HM
             for (int k = threadIdx.x; k < hn; k += BS) {
-                const int j = halo[w * HM + k];
+                double r[XPW];
+                load_row(xp, halo[w * HM + k], r);
+                fast &= row_ok<D>(r);
 #pragma unroll
-                for (int q = 0; q < XPW / 2; q++) {
-                    double a, b;
-                    ld2(xp + (size_t)j * XPW + 2 * q, a, b);
-                    rows[(SORT_WINDOW + k) * (XPW / 2) + q] = make_double2(a, b);
-                }
+                for (int q = 0; q < XPW / 2; q++)
+                    rows[(SORT_WINDOW + k) * (XPW / 2) + q] = make_double2(r[2 * q], r[2 * q + 1]);
             }
         }
-        __syncthreads();
+        fast = __syncthreads_and(fast) != 0;       // every staged row
+    } else {
+        fast &= row_ok<D>(own);
     }
-    if (!live || tag[i] != 0) return;
-
-    double cx[D], vol, xi[D], pv[NF];
-    {
-        if (D == 2) {
-            // the packed row's centroid pair and the dense volume array: 24
-            // bytes per cell less than the 32-byte geometry row
+    const bool real = live && tag[i] == 0;
+    if (!STREAM && !real) return;
+    double out[Y::LD];
+    if (real) {
+        double cx[D], vol, xi[D], pv[NF];
+        {
+            if (D == 2) {
+                // the packed row's centroid pair and the dense volume array: 24
+                // bytes per cell less than the 32-byte geometry row
 #pragma unroll
-            for (int k = 0; k < D; k++) cx[k] = own[XpLay<D>::C + k];
-            vol = vols[i];
-        } else {
-            double g[GEO];
-            ld2(geo + (size_t)i * GEO, g[0], g[1]);
-            ld2(geo + (size_t)i * GEO + 2, g[2], g[3]);
-#pragma unroll
-            for (int k = 0; k < D; k++) cx[k] = g[k];
-            vol = g[3];
-        }
-#pragma unroll
-        for (int k = 0; k < D; k++) xi[k] = own[XpLay<D>::X + k];
-#pragma unroll
-        for (int n = 0; n < NF; n++) pv[n] = own[XpLay<D>::P + n];
-    }
-    double pmax[NF], pmin[NF], df[NF * D];
-#pragma unroll
-    for (int n = 0; n < NF; n++) {
-        pmax[n] = pmin[n] = pv[n];
-#pragma unroll
-        for (int k = 0; k < D; k++) df[n * D + k] = 0.0;
-    }
-    const int deg = off[i + 1] - off[i];
-    const long long base = sbase[t / SLICE] + (t % SLICE);
-    // GB entries in flight: their slot loads, then their row reads, then the
-    // entries applied one by one in list order (the same sums).  Two pay in
-    // 2D; in 3D the extra registers cost a wave per SIMD.  LB: face centroids
-    // in flight in the limiter pass (two measured best in 2D and 3D)
-    constexpr int GB = D == 2 ? 2 : 1, LB = 2;
-    for (int e0 = 0; e0 < deg; e0 += GB) {
-        SlotEnt<D> cur[GB];
-        double rb[GB][XPW];
-#pragma unroll
-        for (int b = 0; b < GB; b++) {
-            cur[b].j = INVALID;
-            if (e0 + b < deg) {
-                const long long slot = base + (long long)(e0 + b) * SLICE;
-                if (HALO) {
-                    // j carries the staged row; LOC_NONE marks an invalid
-                    // neighbour, LOC_GLOBAL one past the staged halo
-                    cur[b] = load_slot<D, false>(sj, sx, sy, sz, sa, slot);
-                    const int loc = __builtin_nontemporal_load(sloc + slot);
-                    cur[b].j = loc == LOC_NONE ? INVALID : loc;
-                } else {
-                    cur[b] = load_slot<D>(sj, sx, sy, sz, sa, slot);
-                }
-            }
-        }
-        if (KC > 0 && e0 < KC) {
-#pragma unroll
-            for (int b = 0; b < GB; b++)
-                if (e0 + b < KC && e0 + b < deg)
-                    ccache[(e0 + b) * SORT_WINDOW + threadIdx.x] = make_double2(cur[b].com[0], cur[b].com[1]);
-        }
-#pragma unroll
-        for (int b = 0; b < GB; b++) {
-            const int j = cur[b].j;
-            if (j == INVALID) continue;
-            const long long lj = (long long)j - w0;
-            if (HALO && j != LOC_GLOBAL) {
-#pragma unroll
-                for (int q = 0; q < XPW / 2; q++) {
-                    const double2 v = rows[j * (XPW / 2) + q];
-                    rb[b][2 * q] = v.x;
-                    rb[b][2 * q + 1] = v.y;
-                }
-            } else if (HALO) {
-                const long long slot = base + (long long)(e0 + b) * SLICE;
-                load_row(xp, sj[slot] & 0x7fffffff, rb[b]);
-            } else if (STAGE && lj >= 0 && lj < SORT_WINDOW) {
-#pragma unroll
-                for (int q = 0; q < XPW / 2; q++) {
-                    const double2 v = rows[lj * (XPW / 2) + q];
-                    rb[b][2 * q] = v.x;
-                    rb[b][2 * q + 1] = v.y;
-                }
+                for (int k = 0; k < D; k++) cx[k] = own[XpLay<D>::C + k];
+                vol = vols[i];
             } else {
-                load_row(xp, j, rb[b]);
+                double g[GEO];
+                ld2(geo + (size_t)i * GEO, g[0], g[1]);
+                ld2(geo + (size_t)i * GEO + 2, g[2], g[3]);
+#pragma unroll
+                for (int k = 0; k < D; k++) cx[k] = g[k];
+                vol = g[3];
             }
+#pragma unroll
+            for (int k = 0; k < D; k++) xi[k] = own[XpLay<D>::X + k];
+#pragma unroll
+            for (int n = 0; n < NF; n++) pv[n] = own[XpLay<D>::P + n];
         }
-#pragma unroll
-        for (int b = 0; b < GB; b++) {
-            if (cur[b].j == INVALID) continue;
-            const double* com = cur[b].com;
-            const double area = cur[b].area;
-            const double* r = rb[b];
-            double cfx[D], dr[D], rr = 0.0;
-#pragma unroll
-            for (int k = 0; k < D; k++) {
-                const double xj = r[XpLay<D>::X + k];
-                cfx[k] = com[k] - 0.5 * (xi[k] + xj);
-                dr[k] = xi[k] - xj;
-                rr += dr[k] * dr[k];
-            }
-            rr = sqrt(rr);
-            const double rv = rr * vol;
-            // Springel (2010) eq. 21 summand, area*(...)/(r*vol) (677-681)
-            double num[NF * D];
-            bool shared = div_operand_ok(rv) & (rv > 0.0);
+        fast &= within(vol, 0x1p-200, 0x1p100);
+        double pmax[NF], pmin[NF], df[NF * D];
+        const int deg = off[i + 1] - off[i];
+        const long long base = sbase[t / SLICE] + (t % SLICE);
+        // The sums over the list, in the arithmetic ar; false when a row that was
+        // not staged, or a distance, is outside the ranges of Shared: the sums are
+        // then formed again with the operators.  (One loop per arithmetic: a branch
+        // per entry holds what both sides share across it.)
+        auto sums = [&](const auto& ar) {
+            constexpr bool SHARED = std::decay_t<decltype(ar)>::fast;
+            bool ok = true;
 #pragma unroll
             for (int n = 0; n < NF; n++) {
-                const double pj = r[XpLay<D>::P + n];
-                pmax[n] = fmax(pmax[n], pj);
-                pmin[n] = fmin(pmin[n], pj);
-                const double d_dif = pj - pv[n];
-                const double d_sum = pj + pv[n];
+                pmax[n] = pmin[n] = pv[n];
 #pragma unroll
-                for (int k = 0; k < D; k++) {
-                    num[n * D + k] = area * (d_dif * cfx[k] - 0.5 * d_sum * dr[k]);
-                    shared &= div_operand_ok(num[n * D + k]);
+                for (int k = 0; k < D; k++) df[n * D + k] = 0.0;
+            }
+            // GB entries in flight: their slot loads, then their row reads, then the
+            // entries applied one by one in list order (the same sums).  128^3: one
+            // 625 us, two 573, three 737 (2 waves per SIMD); 2D ensemble: 484, 421, 463.
+            constexpr int GB = 2;
+            for (int e0 = 0; e0 < deg; e0 += GB) {
+                SlotEnt<D> cur[GB];
+                double rb[GB][XPW];
+#pragma unroll
+                for (int b = 0; b < GB; b++) {
+                    cur[b].j = INVALID;
+                    if (e0 + b < deg) {
+                        const long long slot = base + (long long)(e0 + b) * SLICE;
+                        if (HALO) {
+                            // j carries the staged row; LOC_NONE marks an invalid
+                            // neighbour, LOC_GLOBAL one past the staged halo
+                            cur[b] = load_slot<D, false>(sj, sx, sy, sz, sa, slot);
+                            const int loc = __builtin_nontemporal_load(sloc + slot);
+                            cur[b].j = loc == LOC_NONE ? INVALID : loc;
+                        } else {
+                            cur[b] = load_slot<D>(sj, sx, sy, sz, sa, slot);
+                        }
+                    }
+                }
+                if (KC > 0 && e0 < KC) {
+#pragma unroll
+                    for (int b = 0; b < GB; b++)
+                        if (e0 + b < KC && e0 + b < deg)
+                            ccache[(e0 + b) * SORT_WINDOW + threadIdx.x] = make_double2(cur[b].com[0], cur[b].com[1]);
+                }
+#pragma unroll
+                for (int b = 0; b < GB; b++) {
+                    const int j = cur[b].j;
+                    if (j == INVALID) continue;
+                    const long long lj = (long long)j - w0;
+                    if (HALO ? j != LOC_GLOBAL : (STAGE && lj >= 0 && lj < SORT_WINDOW)) {
+                        const double2* row = rows + (HALO ? (long long)j : lj) * (XPW / 2);
+#pragma unroll
+                        for (int q = 0; q < XPW / 2; q++) {
+                            const double2 v = row[q];
+                            rb[b][2 * q] = v.x;
+                            rb[b][2 * q + 1] = v.y;
+                        }
+                    } else {
+                        const long long slot = base + (long long)(e0 + b) * SLICE;
+                        load_row(xp, HALO ? sj[slot] & 0x7fffffff : j, rb[b]);
+                        if (SHARED) ok &= row_ok<D>(rb[b]);
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < GB; b++) {
+                    if (cur[b].j == INVALID) continue;
+                    const double* com = cur[b].com;
+                    const double area = cur[b].area;
+                    const double* r = rb[b];
+                    double cfx[D], dr[D], rr = 0.0;
+#pragma unroll
+                    for (int k = 0; k < D; k++) {
+                        const double xj = r[XpLay<D>::X + k];
+                        cfx[k] = com[k] - 0.5 * (xi[k] + xj);
+                        dr[k] = xi[k] - xj;
+                        rr += dr[k] * dr[k];
+                    }
+                    if (SHARED) ok &= rr > 0.0;
+                    // Springel (2010) eq. 21 summand, area*(...)/(r*vol) (677-681)
+                    const auto rv = ar.rcp(ar.root(rr) * vol);
+#pragma unroll
+                    for (int n = 0; n < NF; n++) {
+                        const double pj = r[XpLay<D>::P + n];
+                        pmax[n] = fmax(pmax[n], pj);
+                        pmin[n] = fmin(pmin[n], pj);
+                        const double d_dif = pj - pv[n];
+                        const double d_sum = pj + pv[n];
+#pragma unroll
+                        for (int k = 0; k < D; k++)
+                            df[n * D + k] += ar.div(area * (d_dif * cfx[k] - 0.5 * d_sum * dr[k]), rv);
+                    }
                 }
             }
-            if (shared) {
-                const double rcp = rcp_newton(rv);
-#pragma unroll
-                for (int q = 0; q < NF * D; q++) df[q] += div_shared(num[q], rv, rcp);
-            } else {
-#pragma unroll
-                for (int q = 0; q < NF * D; q++) df[q] += num[q] / rv;
-            }
-        }
-    }
+            return ok;
+        };
+        if (fast) fast = sums(Shared());
+        if (!fast) sums(Ieee());
+        // face centroids in flight in the limiter pass (two measured best)
+        constexpr int LB = 2;
 
-    double alpha[NF];
+        double alpha[NF];
 #pragma unroll
-    for (int n = 0; n < NF; n++) alpha[n] = 1.0;
-    if (LIM == PHD_LIMITER_AREPO) {
-        double dpos[NF], dneg[NF];
+        for (int n = 0; n < NF; n++) alpha[n] = 1.0;
+        if (LIM == PHD_LIMITER_AREPO) {
+            double dpos[NF], dneg[NF];
 #pragma unroll
-        for (int n = 0; n < NF; n++) { dpos[n] = 0.0; dneg[n] = 0.0; }
-        for (int e0 = 0; e0 < deg; e0 += LB) {
-            double relb[LB][D];
+            for (int n = 0; n < NF; n++) { dpos[n] = 0.0; dneg[n] = 0.0; }
+            for (int e0 = 0; e0 < deg; e0 += LB) {
+                double relb[LB][D];
 #pragma unroll
-            for (int b = 0; b < LB; b++) {
-                if (e0 + b >= deg) continue;
-                if (KC > 0 && e0 + b < KC) {
-                    const double2 v = ccache[(e0 + b) * SORT_WINDOW + threadIdx.x];
-                    relb[b][0] = v.x - cx[0];
-                    relb[b][1] = v.y - cx[1];
-                    continue;
+                for (int b = 0; b < LB; b++) {
+                    if (e0 + b >= deg) continue;
+                    if (KC > 0 && e0 + b < KC) {
+                        const double2 v = ccache[(e0 + b) * SORT_WINDOW + threadIdx.x];
+                        relb[b][0] = v.x - cx[0];
+                        relb[b][1] = v.y - cx[1];
+                        continue;
+                    }
+                    const long long slot = base + (long long)(e0 + b) * SLICE;
+                    relb[b][0] = __builtin_nontemporal_load(sx + slot) - cx[0];
+                    relb[b][1] = __builtin_nontemporal_load(sy + slot) - cx[1];
+                    if (D == 3) relb[b][D - 1] = __builtin_nontemporal_load(sz + slot) - cx[D - 1];
                 }
-                const long long slot = base + (long long)(e0 + b) * SLICE;
-                relb[b][0] = __builtin_nontemporal_load(sx + slot) - cx[0];
-                relb[b][1] = __builtin_nontemporal_load(sy + slot) - cx[1];
-                if (D == 3) relb[b][D - 1] = __builtin_nontemporal_load(sz + slot) - cx[D - 1];
+#pragma unroll
+                for (int b = 0; b < LB; b++) {
+                    if (e0 + b >= deg) continue;
+#pragma unroll
+                    for (int n = 0; n < NF; n++) {
+                        double dphi = 0.0;
+#pragma unroll
+                        for (int k = 0; k < D; k++) dphi += df[n * D + k] * relb[b][k];
+                        // dpos starts at 0 and only grows, dneg starts at 0 and
+                        // only shrinks, and fmax/fmin skip NaN: the unconditional
+                        // forms leave each one exactly as the reference's
+                        // "dphi > 0" / "dphi < 0" branches do (a -0 is never
+                        // taken as > 0 or < 0 below)
+                        dpos[n] = fmax(dpos[n], dphi);
+                        dneg[n] = fmin(dneg[n], dphi);
+                    }
+                }
             }
 #pragma unroll
-            for (int b = 0; b < LB; b++) {
-                if (e0 + b >= deg) continue;
+            for (int n = 0; n < NF; n++) {
+                if (dpos[n] > 0) alpha[n] = fmin(alpha[n], fmax((pmax[n] - pv[n]) / dpos[n], 0.));
+                if (dneg[n] < 0) alpha[n] = fmin(alpha[n], fmax((pmin[n] - pv[n]) / dneg[n], 0.));
+            }
+        } else {
+            // TESS limiter (reconstruction.pyx:705-731); only alpha[0] changes: the
+            // minimum of all fields' psi over all faces, in any order.  One walk of
+            // the list serves every field, the neighbour's row read as above (a walk
+            // per field with the rows gathered from HBM took 138 us on 41^3, this 68).
+            for (int e = 0; e < deg; e++) {
+                const long long slot = base + (long long)e * SLICE;
+                const double cm[3] = {sx[slot], sy[slot], D == 3 ? sz[slot] : 0.0};
+                int j;
+                double r[XPW];
+                if (HALO) {
+                    const int loc = sloc[slot];
+                    j = loc == LOC_NONE ? INVALID : loc == LOC_GLOBAL ? (sj[slot] & 0x7fffffff) : -1 - loc;
+                } else {
+                    j = sj[slot] & 0x7fffffff;
+                    if (STAGE && j >= w0 && j < w0 + SORT_WINDOW) j = -1 - (int)(j - w0);
+                }
+                if (j == INVALID) continue;
+                if (j < 0) {                   // staged row -1 - j
+#pragma unroll
+                    for (int q = 0; q < XPW / 2; q++) {
+                        const double2 v = rows[(-1 - j) * (XPW / 2) + q];
+                        r[2 * q] = v.x;
+                        r[2 * q + 1] = v.y;
+                    }
+                } else {
+                    load_row(xp, j, r);
+                }
 #pragma unroll
                 for (int n = 0; n < NF; n++) {
                     double dphi = 0.0;
 #pragma unroll
-                    for (int k = 0; k < D; k++) dphi += df[n * D + k] * relb[b][k];
-                    // dpos starts at 0 and only grows, dneg starts at 0 and
-                    // only shrinks, and fmax/fmin skip NaN: the unconditional
-                    // forms leave each one exactly as the reference's
-                    // "dphi > 0" / "dphi < 0" branches do (a -0 is never
-                    // taken as > 0 or < 0 below)
-                    dpos[n] = fmax(dpos[n], dphi);
-                    dneg[n] = fmin(dneg[n], dphi);
+                    for (int k = 0; k < D; k++) dphi += df[n * D + k] * (cm[k] - cx[k]);
+                    double psi;
+                    if (dphi > 0.0 || dphi < 0.0) {
+                        double q = (r[XpLay<D>::P + n] - pv[n]) / dphi;
+                        psi = (0. > q) ? 0. : q;
+                    } else {
+                        psi = 1.0;
+                    }
+                    alpha[0] = fmin(alpha[0], fmax(psi, 0.));
                 }
             }
         }
 #pragma unroll
-        for (int n = 0; n < NF; n++) {
-            if (dpos[n] > 0) alpha[n] = fmin(alpha[n], fmax((pmax[n] - pv[n]) / dpos[n], 0.));
-            if (dneg[n] < 0) alpha[n] = fmin(alpha[n], fmax((pmin[n] - pv[n]) / dneg[n], 0.));
-        }
-    } else {
-        // TESS limiter (reconstruction.pyx:705-731); only alpha[0] changes: the
-        // minimum of all fields' psi over all faces, in any order.  One walk of
-        // the list serves every field, the neighbour's row read as above (a walk
-        // per field with the rows gathered from HBM took 138 us on 41^3, this 68).
-        for (int e = 0; e < deg; e++) {
-            const long long slot = base + (long long)e * SLICE;
-            const double cm[3] = {sx[slot], sy[slot], D == 3 ? sz[slot] : 0.0};
-            int j;
-            double r[XPW];
-            if (HALO) {
-                const int loc = sloc[slot];
-                j = loc == LOC_NONE ? INVALID : loc == LOC_GLOBAL ? (sj[slot] & 0x7fffffff) : -1 - loc;
-            } else {
-                j = sj[slot] & 0x7fffffff;
-                if (STAGE && j >= w0 && j < w0 + SORT_WINDOW) j = -1 - (int)(j - w0);
-            }
-            if (j == INVALID) continue;
-            if (j < 0) {                   // staged row -1 - j
+        for (int n = 0; n < NF; n++) out[Y::P0 + n] = pv[n];
 #pragma unroll
-                for (int q = 0; q < XPW / 2; q++) {
-                    const double2 v = rows[(-1 - j) * (XPW / 2) + q];
-                    r[2 * q] = v.x;
-                    r[2 * q + 1] = v.y;
-                }
-            } else {
-                load_row(xp, j, r);
-            }
+        for (int n = 0; n < NF; n++)
 #pragma unroll
-            for (int n = 0; n < NF; n++) {
-                double dphi = 0.0;
+            for (int k = 0; k < D; k++) out[Y::G0 + n * D + k] = alpha[n] * df[n * D + k];
 #pragma unroll
-                for (int k = 0; k < D; k++) dphi += df[n * D + k] * (cm[k] - cx[k]);
-                double psi;
-                if (dphi > 0.0 || dphi < 0.0) {
-                    double q = (r[XpLay<D>::P + n] - pv[n]) / dphi;
-                    psi = (0. > q) ? 0. : q;
-                } else {
-                    psi = 1.0;
-                }
-                alpha[0] = fmin(alpha[0], fmax(psi, 0.));
-            }
-        }
+        for (int k = 0; k < D; k++) out[Y::C0 + k] = cx[k];
+        if (Y::LD > Y::REC) out[Y::LD - 1] = 0.0;
     }
-    double* row = rec + (size_t)i * ld;
-    double out[Y::LD];
+    if (!STREAM) {
+        double2* row = reinterpret_cast<double2*>(rec + (size_t)i * ld);
 #pragma unroll
-    for (int n = 0; n < NF; n++) out[Y::P0 + n] = pv[n];
+        for (int q = 0; q < Q; q++) row[q] = make_double2(out[2 * q], out[2 * q + 1]);
+        return;
+    }
+    __syncthreads();                               // the rows have been read
+    if (live) written[i - w0] = real;
+    if (real) {
 #pragma unroll
-    for (int n = 0; n < NF; n++)
-#pragma unroll
-        for (int k = 0; k < D; k++) out[Y::G0 + n * D + k] = alpha[n] * df[n * D + k];
-#pragma unroll
-    for (int k = 0; k < D; k++) out[Y::C0 + k] = cx[k];
-    if (Y::LD > Y::REC) out[Y::LD - 1] = 0.0;
-#pragma unroll
-    for (int q = 0; q < Y::LD / 2; q++)
-        reinterpret_cast<double2*>(row)[q] = make_double2(out[2 * q], out[2 * q + 1]);
+        for (int q = 0; q < Q; q++) lds[(i - w0) * Q + q] = make_double2(out[2 * q], out[2 * q + 1]);
+    }
+    __syncthreads();
+    const int nr = (int)min((long long)SORT_WINDOW, n_cells - w0);
+    for (int k = threadIdx.x; k < nr * Q; k += BS) {
+        const int r = k / Q, q = k - r * Q;
+        if (written[r]) reinterpret_cast<double2*>(rec + (size_t)(w0 + r) * ld)[q] = lds[r * Q + q];
+    }
 }
 
 // ghost cell records: gradient copied from the image (domain_manager.pyx:
@@ -1680,7 +1706,7 @@ int launch_grad(phd_handle* h, phd_plan* p, const phd_cells* c, int limiter, dou
         LAUNCHCHK();
     }
     const unsigned nb = xcd_grid(c->n_cells);
-#define GS(L) k_grad_sell<D, L><<<nb, PHD_BLOCK, 0, h->stream>>>(c->n_cells, c->tag, p->cell_geo, c->volume, p->xp, p->off, p->perm, p->sbase, p->sj, p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc, rec, ld)
+#define GS(L) k_grad_sell<D, L><<<nb, PHD_BLOCK, 0, h->stream>>>(c->n_cells, c->tag, p->cell_geo, c->volume, p->xp, p->off, p->perm, p->sbase, p->sj, p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc, p->faces_ok, rec, ld)
     if (limiter == PHD_LIMITER_AREPO) GS(PHD_LIMITER_AREPO);
     else if (limiter == PHD_LIMITER_TESS) GS(PHD_LIMITER_TESS);
     else return PHD_E_MODE;
@@ -2031,8 +2057,8 @@ int phd_plan_create(phd_handle* h, const phd_cells* c, const phd_faces* f, phd_p
         if (hipMemcpyAsync(p->off, f->nbr_off, sizeof(int32_t) * (size_t)(na + 1), hipMemcpyDeviceToDevice, h->stream) != hipSuccess) { rc = PHD_E_HIP; break; }
         k_reset_err<<<1, 64, 0, h->stream>>>(p->d_bad);   // slot 0 = NOERR
         if (nf > 0) {
-            if (D == 2) k_plan_faces<2><<<xcd_grid(nf), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->face_rec);
-            else k_plan_faces<3><<<xcd_grid(nf), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->face_rec);
+            if (D == 2) k_plan_faces<2><<<xcd_grid(nf), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->face_rec, p->d_bad + 2);
+            else k_plan_faces<3><<<xcd_grid(nf), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->face_rec, p->d_bad + 2);
         }
         if (na > 0) {
             if (D == 2) k_plan_cells<2><<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, p->cell_geo, p->xp);
@@ -2041,11 +2067,12 @@ int phd_plan_create(phd_handle* h, const phd_cells* c, const phd_faces* f, phd_p
             k_plan_runs<<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, p->csr, p->off, p->d_bad + 1);
         }
         if (hipPeekAtLastError() != hipSuccess) { (void)hipGetLastError(); rc = PHD_E_HIP; break; }
-        unsigned long long bad[2] = {NOERR, NOERR};
+        unsigned long long bad[3] = {NOERR, NOERR, NOERR};
         if (hipMemcpyAsync(bad, p->d_bad, sizeof(bad), hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
             hipStreamSynchronize(h->stream) != hipSuccess) { rc = PHD_E_HIP; break; }
         p->bad_cell = bad[0] == NOERR ? -1 : (long long)bad[0];
         p->owner_runs = bad[1] == NOERR;
+        p->faces_ok = bad[2] == NOERR;
         rc = build_slots(h, p, c, f);
         if (!rc) rc = build_halo(h, p, c);
         if (!rc) rc = build_ghost_list(h, p, c);
@@ -2450,7 +2477,7 @@ int batch_grad(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_schedul
         k_grad_sell<D, PHD_LIMITER_AREPO, BS, XC><<<sched_grid<BS, XC>(n), BS, 0, h->stream>>>( \
             c->n_cells, c->tag, p->cell_geo, c->volume, p->xp, p->off, p->perm, p->sbase,      \
             p->sj, p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc,  \
-            rec, ld);                                                                          \
+            p->faces_ok, rec, ld);                                                                          \
         LAUNCHCHK();                                                                           \
         return 0;                                                                              \
     }

@@ -65,3 +65,34 @@ def test_fused_fluxes_equal_materialised(gpu, dim, n, scale):
                     x, y = x.cpu().numpy(), y.cpu().numpy()
                     same = (x.view(np.int64) == y.view(np.int64)) | (np.isnan(x) & np.isnan(y))
                     assert same.all(), (solver, boost, gizmo, q, int((~same).sum()))
+
+
+@pytest.mark.parametrize("limiter", [0, 1])
+@pytest.mark.parametrize("scale", [0, 60, 99, 130, 300])
+@pytest.mark.parametrize("name,n", [("kh_2d", 33), ("sod_2d", 4), ("sedov_3d", 11)])
+def test_gradients_equal_oracle_over_scales(gpu, name, n, scale, limiter):
+    """Primitives in and past the ranges Shared takes, zeros among them, in a
+    third of the windows' cells: the limited gradients bit for bit."""
+    from oracle import oracle
+    from phd import problems
+    from parity import assert_bitwise
+    print("case gradients %s n=%d scale 2^+-%d limiter %d" % (name, n, scale, limiter), flush=True)
+    p = problems.PROBLEMS[name](n=n, seed=1)
+    pc = p.particles
+    na = pc.get_carray_size()
+    rng = np.random.default_rng(scale + n)
+    for q, f in enumerate(pc.carray_named_groups["primitive"]):
+        v = rng.uniform(0.5, 2.0, na) if q in (0, p.dim + 1) else rng.normal(0, 1, na)
+        some = rng.random(na) < 0.01
+        v[some] *= 2.0 ** rng.integers(-scale, scale + 1, some.sum())
+        v[rng.random(na) < 0.05] = 0.0
+        pc[f][:] = torch.as_tensor(v, device=gpu)
+    a = problems.host_arrays(p)
+    p.recon.slope_limiter = limiter
+    p.recon.compute_gradients(pc, p.mesh, p.domain_manager)
+    grad, rc, _ = oracle.compute_gradients(a, limiter)
+    assert rc == 0
+    real = a["tag"] == 0
+    got = p.recon.grad.rows().cpu().numpy()
+    for q in range(len(grad)):
+        assert_bitwise(got[real, q], grad[q][real], "grad %d" % q)
