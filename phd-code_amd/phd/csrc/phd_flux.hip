@@ -287,6 +287,8 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_plan_runs(phd_cells c, const int2
 constexpr int SLICE = 16;
 constexpr int SORT_WINDOW = PHD_BLOCK;   // cells per degree-sorted window
 
+inline long long n_windows(const phd_cells* c) { return ((long long)c->n_cells + SORT_WINDOW - 1) / SORT_WINDOW; }
+
 // width of each 16-cell slice = the largest face-list length of its real cells
 // position -> cell order: inside each window of SORT_WINDOW consecutive
 // cells, real cells by descending face count (ties by id), then ghosts
@@ -1290,6 +1292,11 @@ __global__ __launch_bounds__(BS) void k_update_sell(phd_cells c, const double* _
 // gathered.  CAP rows leave two blocks a CU their LDS in 3D (about 2020 faces a
 // window) and five in 2D (768).  Against a walk of the CSR entries one by one:
 // 512^2 in 2D 41 -> 28 us, 41^3 54 -> 39 us.
+// Fewer windows than flux_stage_min leave CUs idle, and the staging is then one
+// more latency of the few blocks there are (staged and not: 150^2 11.2 and 8.1 us,
+// 256^2 14.4 and 12.5, 400^2 16.6 and 18.8; 30^3 32 and 28, 41^3 38 and 50); in 3D
+// 64-thread blocks then spread the gathers over more CUs (21^3 26 -> 20 us).
+template <int D> constexpr int flux_stage_min() { return D == 2 ? 512 : 256; }
 template <int D> constexpr int flux_cap() { return D == 2 ? 800 : 1750; }
 
 struct StagedSummands {
@@ -1308,8 +1315,8 @@ struct StagedSummands {
     }
 };
 
-template <int D, int OR>
-__global__ __launch_bounds__(PHD_BLOCK) void k_update_flux(phd_cells c, int n_faces,
+template <int D, int OR, int STAGED, int BS>
+__global__ __launch_bounds__(BS) void k_update_flux(phd_cells c, int n_faces,
                                                            FluxSummands src,
                                                            const int2* __restrict__ csr,
                                                            const int32_t* __restrict__ off,
@@ -1319,7 +1326,7 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_update_flux(phd_cells c, int n_fa
                                                            const int2* __restrict__ cinfo,
                                                            unsigned long long* err)
 {
-    if constexpr (OR) {
+    if constexpr (STAGED) {
         __shared__ double rows[flux_cap<D>() * (D + 2)];
         __shared__ int first;
         const long long t = xcd_index(c.n_cells);
@@ -1341,7 +1348,7 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_update_flux(phd_cells c, int n_fa
         update_body<D, PHD_BLOCK, 1, OR>(c, StagedSummands{src, rows, f0, n}, csr, off, perm, sbase,
                                          sfi, cinfo, err);
     } else {
-        update_body<D, PHD_BLOCK, 1, OR>(c, src, csr, off, perm, sbase, sfi, cinfo, err);
+        update_body<D, BS, 1, OR>(c, src, csr, off, perm, sbase, sfi, cinfo, err);
     }
 }
 
@@ -1780,14 +1787,21 @@ int launch_face(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces*
     return PHD_E_MODE;
 }
 
+// A 3D cell's rows are 80 uncoalesced loads, and the waves of one block share a
+// CU's address unit: a mesh of few blocks is updated by 64-thread blocks, which
+// spread over four times the CUs (21^3 14.5 -> 11.5 us, 41^3 22.8 -> 20.4; 2D,
+// with a fifth of the loads, gains nothing).
+template <int D> constexpr int small_update() { return D == 3 ? 512 : 0; }
+
 template <int D>
 int launch_update(phd_handle* h, phd_plan* p, const phd_cells* c)
 {
     if (c->n_cells == 0) return 0;
-#define US(OR) k_update_sell<D, PHD_BLOCK, 1, OR><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, p->g, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
-    if (p->owner_runs) US(1);
-    else US(0);
-#undef US
+#define UB(OR, BS) k_update_sell<D, BS, 1, OR><<<sched_grid<BS, 1>(c->n_cells), BS, 0, h->stream>>>(*c, p->g, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
+    if (!p->owner_runs) UB(0, PHD_BLOCK);
+    else if (n_windows(c) < small_update<D>()) UB(1, 64);
+    else UB(1, PHD_BLOCK);
+#undef UB
     LAUNCHCHK();
     return 0;
 }
@@ -1796,9 +1810,11 @@ template <int D>
 int launch_update_flux(phd_handle* h, phd_plan* p, const phd_cells* c, const FluxSummands& src)
 {
     if (c->n_cells == 0) return 0;
-#define UF(OR) k_update_flux<D, OR><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, p->n_faces, src, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
-    if (p->owner_runs) UF(1);
-    else UF(0);
+#define UF(OR, ST, BS) k_update_flux<D, OR, ST, BS><<<sched_grid<BS, 1>(c->n_cells), BS, 0, h->stream>>>(*c, p->n_faces, src, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
+    if (!p->owner_runs) UF(0, 0, PHD_BLOCK);
+    else if (n_windows(c) >= flux_stage_min<D>()) UF(1, 1, PHD_BLOCK);
+    else if (D == 3) UF(1, 0, 64);
+    else UF(1, 0, PHD_BLOCK);
 #undef UF
     LAUNCHCHK();
     return 0;
