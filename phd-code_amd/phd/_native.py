@@ -204,28 +204,36 @@ def mesh_lib():
     return _mesh
 
 
+_gpu_seen = False
+
+
 def flux():
-    """The HIP library, for compute calls: needs a visible GPU."""
-    if not torch.cuda.is_available():
-        raise NativeUnavailable(
-            "phd: the face-flux pipeline runs only on the GPU through libphd_flux.so "
-            "and no GPU is visible (torch.cuda.is_available() is False)")
-    return load_flux_library()
+    """The HIP library, for compute calls: needs a visible GPU (a GPU that has
+    been seen stays; the question costs 2 us and a step asks it 18 times)."""
+    global _gpu_seen
+    if not _gpu_seen:
+        if not torch.cuda.is_available():
+            raise NativeUnavailable(
+                "phd: the face-flux pipeline runs only on the GPU through libphd_flux.so "
+                "and no GPU is visible (torch.cuda.is_available() is False)")
+        _gpu_seen = True
+    return _flux if _flux is not None else load_flux_library()
 
 
 def handle(device=None):
     """Per-device library handle, with its stream set to torch's current one."""
     lib = flux()
-    dev = torch.cuda.current_device() if device is None else int(device)
+    dev = torch._C._cuda_getDevice() if device is None else int(device)
     h = _handles.get(dev)
     if h is None:
+        torch.cuda.init()
         hp = c_vp()
         rc = lib.phd_handle_create(ctypes.byref(hp), dev)
         if rc != 0:
             raise RuntimeError("phd_handle_create failed: %s" % lib.phd_error_string(rc).decode())
         h = hp.value
         _handles[dev] = h
-    lib.phd_set_stream(h, c_vp(torch.cuda.current_stream(dev).cuda_stream))
+    lib.phd_set_stream(h, torch._C._cuda_getCurrentRawStream(dev))
     return h
 
 

@@ -99,7 +99,14 @@ class CarrayContainer(object):
         self._compact(self["tag"] != tag)
 
     def _compact(self, keep):
-        n = int(keep.sum().item())
+        # the items kept, and how often a kept one follows a dropped one: never
+        # when the kept ones come first (dropping the ghosts, which are
+        # appended), and the arrays stay as they are
+        later = keep[1:] & ~keep[:-1]
+        n, moved = torch.stack((keep.sum(), later.sum())).tolist()
+        if moved == 0:
+            self._size = n
+            return
         for name, t in self.carrays.items():
             t[:n] = t[:self._size][keep]
         self._size = n
@@ -110,7 +117,7 @@ class CarrayContainer(object):
         out = CarrayContainer(device=self.device)
         out._size = out._cap = int(idx.numel())
         for name in names:
-            out.carrays[name] = self.carrays[name][:self._size][idx].clone()
+            out.carrays[name] = self.carrays[name][:self._size][idx]
             out.carray_dtypes[name] = self.carray_dtypes[name]
         out.carray_named_groups = {k: list(v) for k, v in self.carray_named_groups.items()}
         return out

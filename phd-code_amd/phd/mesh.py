@@ -143,7 +143,19 @@ class Mesh(object):
                             geometry=not self.device_geometry)
         ng = geo["ghost_map"].size
         dev = particles.device
-        if ng:
+        if ng and "map" in particles.carrays and dev.type == "cuda":
+            # room for the ghosts, then one pass over all fields takes them
+            # from their images (extract and append are two calls per field)
+            particles.extend(ng)
+            particles["tag"][n:] = ParticleTAGS.Ghost
+            particles["map"][n:] = torch.as_tensor(geo["ghost_map"], device=dev)
+            domain_manager.update_ghost_fields(
+                particles, [f for f in particles.carrays if f not in ("tag", "map")])
+            particles["type"][n:] = ParticleTAGS.Exterior
+            if not self.device_geometry:
+                for k, f in enumerate(particles.carray_named_groups["position"]):
+                    particles[f][n:] = torch.as_tensor(geo["ghost_x"][k], device=dev)
+        elif ng:
             gmap = torch.as_tensor(geo["ghost_map"], device=dev, dtype=torch.long)
             ghosts = particles.extract_items(gmap)
             if not self.device_geometry:
