@@ -47,8 +47,11 @@ namespace {
 template <int D> constexpr int pg_width() { return Lay<D>::NF + Lay<D>::G; }
 template <int D> constexpr int frow_width() { return 2 * pg_width<D>(); }
 
-__global__ __launch_bounds__(PHD_BLOCK) void k_adj_mirror(int n_cells, const int2* csr,
-                                                          const int32_t* off, int32_t* mirror)
+// Per list entry, the place of the same face in the other cell's list, or -1
+// where that cell writes no contribution (an invalid neighbour or a ghost)
+__global__ __launch_bounds__(PHD_BLOCK) void k_adj_mirror(int n_cells, const int8_t* tag,
+                                                          const int2* csr, const int32_t* off,
+                                                          int32_t* mirror)
 {
     long long c = xcd_index(n_cells);
     if (c >= n_cells) return;
@@ -56,7 +59,7 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_mirror(int n_cells, const int
         const int2 en = csr[e];
         const int o = en.y & 0x7fffffff;
         int pos = -1;
-        if (o != INVALID) {
+        if (o != INVALID && tag[o] == 0) {
             int lo = off[o], hi = off[o + 1] - 1;
             while (lo <= hi) {       // lists are ascending in face id
                 const int mid = (lo + hi) >> 1;
@@ -185,20 +188,39 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_face_b(phd_cells c, phd_faces
     for (int q = 0; q < W / 2; q++) o[q] = make_double2(row[2 * q], row[2 * q + 1]);
 }
 
+// The face list of the cell at sliced position t: entry e's neighbour row from
+// the block's staging (the window's rows, then its halo; from HBM past it) and
+// its face's centroid and area from the slot arrays, coalesced.
 template <int D>
-struct CsrNbr {
-    const int2* csr;
-    int beg, n;
+struct SellNbr {
+    int n;
+    long long base;                        // slot of entry 0
+    const double2* rows;
     const double* xp;
-    const double* frec;
-    double* contrib;
+    const int32_t* sj;
+    const uint16_t* sloc;
+    const double* const* sgeo;
+    double* out_rows;                      // the cell's contrib rows
     PHD_HD int deg() const { return n; }
-    PHD_HD bool valid(int e) const { return (csr[beg + e].y & 0x7fffffff) != INVALID; }
+    PHD_HD long long slot(int e) const { return base + (long long)e * 16; }
+    PHD_HD bool valid(int e) const { return sloc[slot(e)] != LOC_NONE; }
     PHD_HD void row(int e, double* r) const
     {
-        const int o = csr[beg + e].y & 0x7fffffff;
+        const int loc = sloc[slot(e)];
+        double s[XPW];
+        if (loc != LOC_GLOBAL) {
+#pragma unroll
+            for (int q = 0; q < XPW / 2; q++) {
+                const double2 v = rows[loc * (XPW / 2) + q];
+                s[2 * q] = v.x;
+                s[2 * q + 1] = v.y;
+            }
+        } else {
+            const int j = sj[slot(e)] & 0x7fffffff;
+#pragma unroll
+            for (int q = 0; q < XPW; q++) s[q] = xp[(size_t)j * XPW + q];
+        }
         // as [position | primitive], the order grad_cell_vjp reads
-        const double* s = xp + (size_t)o * XPW;
 #pragma unroll
         for (int k = 0; k < D; k++) r[k] = s[XpLay<D>::X + k];
 #pragma unroll
@@ -206,17 +228,16 @@ struct CsrNbr {
     }
     PHD_HD void geo(int e, double* cm, double& a) const
     {
-        using F = FrLay<D>;
-        const double* fr = frec + (size_t)csr[beg + e].x * F::W;
-        cm[0] = fr[F::C];
-        cm[1] = fr[F::C + 1];
-        cm[2] = D == 3 ? fr[F::C + 2] : 0.0;
-        a = fr[F::A];
+        const long long k = slot(e);
+        cm[0] = sgeo[0][k];
+        cm[1] = sgeo[1][k];
+        cm[2] = D == 3 ? sgeo[2][k] : 0.0;
+        a = sgeo[3][k];
     }
     PHD_HD void out(int e, const double* lam) const
     {
 #pragma unroll
-        for (int q = 0; q < D + 2; q++) contrib[(size_t)(beg + e) * (D + 2) + q] = lam[q];
+        for (int q = 0; q < D + 2; q++) out_rows[(size_t)e * (D + 2) + q] = lam[q];
     }
 };
 
@@ -228,12 +249,56 @@ __device__ __forceinline__ void gather_rows(int cc, const int2* __restrict__ csr
                                             const double* __restrict__ frow, double* s)
 {
     constexpr int PW = pg_width<D>(), W = frow_width<D>();
-    for (int e = off[cc]; e < off[cc + 1]; e++) {
-        const int2 en = csr[e];
-        if ((en.y & 0x7fffffff) == INVALID) continue;
-        const double* r = frow + (size_t)en.x * W + ((en.y & INCOMING) ? PW : 0);
+    constexpr int B = D == 2 ? 3 : 2;
+    const int beg = off[cc], end = off[cc + 1];
+    for (int e0 = beg; e0 < end; e0 += B) {
+        int2 en[B];
+        double2 r[B][PW / 2];
 #pragma unroll
-        for (int q = 0; q < PW; q++) s[q] += r[q];
+        for (int b = 0; b < B; b++) en[b] = e0 + b < end ? csr[e0 + b] : make_int2(0, INVALID);
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            if ((en[b].y & 0x7fffffff) == INVALID) continue;
+            const double2* p = reinterpret_cast<const double2*>(
+                frow + (size_t)en[b].x * W + ((en[b].y & INCOMING) ? PW : 0));
+#pragma unroll
+            for (int q = 0; q < PW / 2; q++) r[b][q] = p[q];
+        }
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            if ((en[b].y & 0x7fffffff) == INVALID) continue;
+#pragma unroll
+            for (int q = 0; q < PW / 2; q++) { s[2 * q] += r[b][q].x; s[2 * q + 1] += r[b][q].y; }
+        }
+    }
+}
+
+// The same over the cell's sliced list (face ids coalesced), B rows in flight
+template <int D>
+__device__ __forceinline__ void gather_slots(long long base, int deg,
+                                             const int32_t* __restrict__ sfi,
+                                             const double* __restrict__ frow, double* s)
+{
+    constexpr int PW = pg_width<D>(), W = frow_width<D>(), B = D == 2 ? 3 : 2;
+    for (int e0 = 0; e0 < deg; e0 += B) {
+        int en[B];
+        double2 r[B][PW / 2];
+#pragma unroll
+        for (int b = 0; b < B; b++) en[b] = e0 + b < deg ? sfi[base + (long long)(e0 + b) * 16] : INVALID;
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            if (en[b] == INVALID) continue;
+            const double2* p = reinterpret_cast<const double2*>(
+                frow + (size_t)(en[b] & 0x7fffffff) * W + ((en[b] & INCOMING) ? PW : 0));
+#pragma unroll
+            for (int q = 0; q < PW / 2; q++) r[b][q] = p[q];
+        }
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            if (en[b] == INVALID) continue;
+#pragma unroll
+            for (int q = 0; q < PW / 2; q++) { s[2 * q] += r[b][q].x; s[2 * q + 1] += r[b][q].y; }
+        }
     }
 }
 
@@ -243,56 +308,100 @@ __device__ __forceinline__ void gather_rows(int cc, const int2* __restrict__ csr
 // grad_k with d v_q / d x_q negated); then the gradient VJP: lself gets the
 // primitives' total (faces + own gradient), contrib one vector per list
 // entry for the entry's other cell
+//
+// One block per window, as the gradient kernel, with its staged rows and sliced
+// lists: three walks of the CSR list, each entry two dependent gathers, took 41
+// us at 256^2 and 130 at 21^3, this 38 and 94.
 template <int D>
-__global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, int n_real,
-                                                        const int2* __restrict__ csr,
+__global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2* __restrict__ csr,
                                                         const int32_t* __restrict__ off,
+                                                        const int32_t* __restrict__ perm,
+                                                        const int32_t* __restrict__ sbase,
+                                                        const int32_t* __restrict__ sj,
+                                                        const int32_t* __restrict__ sfi,
+                                                        const double* __restrict__ sx,
+                                                        const double* __restrict__ sy,
+                                                        const double* __restrict__ sz,
+                                                        const double* __restrict__ sa,
+                                                        const int32_t* __restrict__ hcnt,
+                                                        const int32_t* __restrict__ halo,
+                                                        const uint16_t* __restrict__ sloc,
+                                                        int faces_ok,
                                                         const int32_t* __restrict__ gofs,
                                                         const int32_t* __restrict__ gids,
                                                         int reflect, double lo0, double lo1,
                                                         double lo2, double hi0, double hi1,
                                                         double hi2, const double* __restrict__ xp,
                                                         const double* __restrict__ geo,
-                                                        const double* __restrict__ frec,
                                                         const double* __restrict__ frow,
                                                         double* __restrict__ contrib,
                                                         double* __restrict__ lself)
 {
     using Y = Lay<D>;
-    constexpr int NF = Y::NF, PW = pg_width<D>();
-    long long ii = xcd_index(n_real);
-    if (ii >= n_real) return;
-    const int i = (int)ii;
+    constexpr int NF = Y::NF, PW = pg_width<D>(), HM = halo_max<D>();
+    __shared__ double2 rows[(PHD_BLOCK + HM) * XPW / 2];
+    const long long t = xcd_index(c.n_cells);
+    const bool live = t < c.n_cells;
+    const long long w0 = t - threadIdx.x;
+    const int i = live ? perm[t] : 0;
+    bool fast = faces_ok != 0;
+    auto stage = [&](long long cell, int at) {
+        double r[XPW];
+#pragma unroll
+        for (int q = 0; q < XPW / 2; q++) ld2(xp + (size_t)cell * XPW + 2 * q, r[2 * q], r[2 * q + 1]);
+        fast &= row_ok<D>(r);
+#pragma unroll
+        for (int q = 0; q < XPW / 2; q++) rows[at * (XPW / 2) + q] = make_double2(r[2 * q], r[2 * q + 1]);
+    };
+    if (live) stage(t, threadIdx.x);
+    if (w0 < c.n_cells) {
+        const long long w = w0 / PHD_BLOCK;
+        const int hn = hcnt[w];
+        for (int k = threadIdx.x; k < hn; k += PHD_BLOCK) stage(halo[w * HM + k], PHD_BLOCK + k);
+    }
+    fast = __syncthreads_and(fast) != 0;
+    if (!live || c.tag[i] != 0) return;
     const double lo[3] = {lo0, lo1, lo2}, hi[3] = {hi0, hi1, hi2};
+    const int beg = off[i], deg = off[i + 1] - beg;
+    const long long base = sbase[t / 16] + (t % 16);
     double s[PW];
 #pragma unroll
     for (int q = 0; q < PW; q++) s[q] = 0.0;
-    gather_rows<D>(i, csr, off, frow, s);
+    gather_slots<D>(base, deg, sfi, frow, s);
     for (int a = gofs[i]; a < gofs[i + 1]; a++) {
         const int g = gids[a];
         const int fl = ghost_flips<D>(c, g, reflect, lo, hi);
-        double t[PW];
+        double u[PW];
 #pragma unroll
-        for (int q = 0; q < PW; q++) t[q] = 0.0;
-        gather_rows<D>(g, csr, off, frow, t);
+        for (int q = 0; q < PW; q++) u[q] = 0.0;
+        gather_rows<D>(g, csr, off, frow, u);
 #pragma unroll
         for (int q = 0; q < D; q++) {
             if (fl & (1 << q)) {
-                t[1 + q] = -t[1 + q];
-                t[NF + (1 + q) * D + q] = -t[NF + (1 + q) * D + q];
+                u[1 + q] = -u[1 + q];
+                u[NF + (1 + q) * D + q] = -u[NF + (1 + q) * D + q];
             }
         }
 #pragma unroll
-        for (int q = 0; q < PW; q++) s[q] += t[q];
+        for (int q = 0; q < PW; q++) s[q] += u[q];
     }
-    double pv[NF], xi[D], cx[D], vol;
+    double pv[NF], xi[D], cx[D], own[XPW];
 #pragma unroll
-    for (int q = 0; q < NF; q++) pv[q] = xp[(size_t)i * XPW + XpLay<D>::P + q];
+    for (int q = 0; q < XPW / 2; q++) {
+        const double2 v = rows[(i - w0) * (XPW / 2) + q];
+        own[2 * q] = v.x;
+        own[2 * q + 1] = v.y;
+    }
 #pragma unroll
-    for (int k = 0; k < D; k++) { xi[k] = xp[(size_t)i * XPW + XpLay<D>::X + k]; cx[k] = geo[(size_t)i * GEO + k]; }
-    vol = geo[(size_t)i * GEO + 3];
-    CsrNbr<D> nb{csr, off[i], off[i + 1] - off[i], xp, frec, contrib};
-    grad_cell_vjp<D>(nb, pv, xi, cx, vol, s + NF, s);
+    for (int q = 0; q < NF; q++) pv[q] = own[XpLay<D>::P + q];
+#pragma unroll
+    for (int k = 0; k < D; k++) { xi[k] = own[XpLay<D>::X + k]; cx[k] = geo[(size_t)i * GEO + k]; }
+    const double vol = geo[(size_t)i * GEO + 3];
+    const double* const sg[4] = {sx, sy, sz, sa};
+    const SellNbr<D> nb{deg, base, rows, xp, sj, sloc, sg, contrib + (size_t)beg * NF};
+    // a row past the staging was not checked
+    for (int e = 0; e < deg; e++) fast &= sloc[base + (long long)e * 16] != LOC_GLOBAL;
+    grad_cell_vjp<D>(nb, pv, xi, cx, vol, s + NF, s, fast & within(vol, 0x1p-200, 0x1p100));
 #pragma unroll
     for (int q = 0; q < NF; q++) lself[(size_t)i * NF + q] = s[q];
 }
@@ -300,7 +409,6 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, int n_real,
 // K3
 template <int D>
 __global__ __launch_bounds__(PHD_BLOCK) void k_adj_combine(phd_cells c, int n_real,
-                                                           const int2* __restrict__ csr,
                                                            const int32_t* __restrict__ off,
                                                            const int32_t* __restrict__ mirror,
                                                            const int32_t* __restrict__ gofs,
@@ -322,21 +430,34 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_combine(phd_cells c, int n_re
 #pragma unroll
     for (int q = 0; q < NF; q++) lp[q] = lself[(size_t)k * NF + q];
     // neighbours' gradient VJPs that read this cell's primitives
-    for (int e = off[k]; e < off[k + 1]; e++) {
-        const int o = csr[e].y & 0x7fffffff;
-        const int src = mirror[e];
-        if (o == INVALID || src < 0 || c.tag[o] != 0) continue;
+    // (eight entries in flight)
+    constexpr int B = 8;
+    const int beg = off[k], end = off[k + 1];
+    for (int e0 = beg; e0 < end; e0 += B) {
+        int src[B];
+        double r[B][NF];
 #pragma unroll
-        for (int q = 0; q < NF; q++) lp[q] += contrib[(size_t)src * NF + q];
+        for (int b = 0; b < B; b++) src[b] = e0 + b < end ? mirror[e0 + b] : -1;
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            if (src[b] < 0) continue;
+#pragma unroll
+            for (int q = 0; q < NF; q++) r[b][q] = contrib[(size_t)src[b] * NF + q];
+        }
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            if (src[b] < 0) continue;
+#pragma unroll
+            for (int q = 0; q < NF; q++) lp[q] += r[b][q];
+        }
     }
     // ... and those that read a ghost copy of it
     for (int a = gofs[k]; a < gofs[k + 1]; a++) {
         const int g = gids[a];
         const int fl = ghost_flips<D>(c, g, reflect, lo, hi);
         for (int e = off[g]; e < off[g + 1]; e++) {
-            const int o = csr[e].y & 0x7fffffff;
             const int src = mirror[e];
-            if (o == INVALID || src < 0 || c.tag[o] != 0) continue;
+            if (src < 0) continue;
             double t[NF];
 #pragma unroll
             for (int q = 0; q < NF; q++) t[q] = contrib[(size_t)src * NF + q];
@@ -425,11 +546,12 @@ int step_vjp(phd_handle* h, phd_plan* p, phd_adjoint* a, const phd_cells* c, con
         else ADJ_FACES(3);
 #undef ADJ_FACES
     }
-    k_adj_cell<D><<<xcd_grid(a->n_real), PHD_BLOCK, 0, h->stream>>>(
-        *c, a->n_real, p->csr, p->off, a->gofs, a->gids, refl, l[0], l[1], l[2], u[0], u[1], u[2],
-        p->xp, p->cell_geo, p->face_rec, a->frow, a->contrib, a->lself);
+    k_adj_cell<D><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(
+        *c, p->csr, p->off, p->perm, p->sbase, p->sj, p->sfi, p->sgeo[0], p->sgeo[1], p->sgeo[2],
+        p->sgeo[3], p->hcnt, p->halo, p->sloc, p->faces_ok, a->gofs, a->gids, refl, l[0], l[1], l[2], u[0], u[1],
+        u[2], p->xp, p->cell_geo, a->frow, a->contrib, a->lself);
     k_adj_combine<D><<<xcd_grid(a->n_real), PHD_BLOCK, 0, h->stream>>>(
-        *c, a->n_real, p->csr, p->off, a->mirror, a->gofs, a->gids, refl, l[0], l[1], l[2], u[0],
+        *c, a->n_real, p->off, a->mirror, a->gofs, a->gids, refl, l[0], l[1], l[2], u[0],
         u[1], u[2], a->lself, a->contrib, gamma, Lo, Li);
     ADJ_CHK();
     return 0;
@@ -492,7 +614,7 @@ int phd_adjoint_create(phd_handle* h, phd_plan* p, const phd_cells* c, const phd
     if (ok && !gids.empty())
         ok = hipMemcpyAsync(a->gids, gids.data(), 4 * gids.size(), hipMemcpyHostToDevice, h->stream) == hipSuccess;
     if (ok && na > 0) {
-        k_adj_mirror<<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>((int)na, p->csr, p->off, a->mirror);
+        k_adj_mirror<<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>((int)na, c->tag, p->csr, p->off, a->mirror);
         ok = hipPeekAtLastError() == hipSuccess;
     }
     ok = ok && hipStreamSynchronize(h->stream) == hipSuccess;

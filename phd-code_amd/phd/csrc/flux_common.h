@@ -228,6 +228,34 @@ __device__ __forceinline__ void ld2(const double* p, double& a, double& b)
     b = v.y;
 }
 
+// x == 0 or |x| in [2^-100, 2^100]; false for inf and NaN (non-short-circuit
+// operators: the test compiles to compares and mask logic, no branches)
+__device__ __forceinline__ bool operand_ok(double x)
+{
+    const double ax = fabs(x);
+    return (ax <= 0x1p100) & ((ax >= 0x1p-100) | (x == 0.0));
+}
+
+// Ranges of the gradient sums' operands, for the Shared arithmetic (quot_dev.h).
+// With every position, primitive, face centroid and area zero or in [2^-100,
+// 2^100] and volumes in [2^-200, 2^100]: differences and sums of them are zero
+// or >= 2^-153, the distance r = sqrt(sum dr^2) lies in [2^-153, 2^102] unless
+// zero, r * vol in [2^-353, 2^202], and the numerators area * (...) are zero or
+// in [2^-459, 2^304].  So the values are checked once, where a row is staged and
+// (the faces) where the plan is made, and not the numerators of every entry.
+//
+// row_ok: every value of a packed row that the gradients take
+template <int D>
+__device__ __forceinline__ bool row_ok(const double* r)
+{
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < D; k++) ok &= operand_ok(r[XpLay<D>::X + k]);
+#pragma unroll
+    for (int n = 0; n < D + 2; n++) ok &= operand_ok(r[XpLay<D>::P + n]);
+    return ok;
+}
+
 template <int D>
 __device__ __forceinline__ void load_face_rec(const double* frec, long long m, double* com,
                                               double& area, double* n, double& diff)

@@ -5,6 +5,7 @@
 #include <string.h>
 #include "riemann_dev.h"
 #include "states_dev.h"
+#include "adjoint_dev.h"
 
 using namespace phd;
 
@@ -55,4 +56,42 @@ extern "C" void qh_faces(int dim, int hllc, long nf, const double* ri, const dou
     else if (dim == 2) faces<2, PHD_SOLVER_HLL>(nf, ri, rj, com, diff, n, fv, gamma, dt, boost, gizmo, ok, same);
     else if (hllc) faces<3, PHD_SOLVER_HLLC>(nf, ri, rj, com, diff, n, fv, gamma, dt, boost, gizmo, ok, same);
     else faces<3, PHD_SOLVER_HLL>(nf, ri, rj, com, diff, n, fv, gamma, dt, boost, gizmo, ok, same);
+}
+
+namespace {
+
+template <int D>
+struct List {
+    int n;
+    const double *rows, *com, *area;
+    double* lnb;
+    int deg() const { return n; }
+    bool valid(int e) const { return area[e] >= 0.0; }
+    void row(int e, double* r) const { for (int q = 0; q < 8; q++) r[q] = rows[8 * e + q]; }
+    void geo(int e, double* c, double& a) const
+    {
+        for (int k = 0; k < 3; k++) c[k] = com[3 * e + k];
+        a = area[e];
+    }
+    void out(int e, const double* lam) const { for (int q = 0; q < D + 2; q++) lnb[(D + 2) * e + q] = lam[q]; }
+};
+
+template <int D>
+void grad(int deg, const double* rows, const double* com, const double* area, const double* pv,
+          const double* xi, const double* cx, double vol, const double* lgrad, int fast,
+          double* lself, double* lnb)
+{
+    List<D> l{deg, rows, com, area, lnb};
+    grad_cell_vjp<D>(l, pv, xi, cx, vol, lgrad, lself, fast != 0);
+}
+
+} // namespace
+
+extern "C" void qh_grad_vjp(int dim, int deg, const double* rows, const double* com,
+                            const double* area, const double* pv, const double* xi,
+                            const double* cx, double vol, const double* lgrad, int fast,
+                            double* lself, double* lnb)
+{
+    if (dim == 2) grad<2>(deg, rows, com, area, pv, xi, cx, vol, lgrad, fast, lself, lnb);
+    else grad<3>(deg, rows, com, area, pv, xi, cx, vol, lgrad, fast, lself, lnb);
 }

@@ -18,7 +18,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "phd-code_amd", "phd", "csrc")
 SRC = os.path.join(ROOT, "tests", "quotients", "quot_host.cpp")
 LIB = os.path.join(ROOT, "tests", "quotients", "libquot_host.so")
-DEPS = [SRC] + [os.path.join(CSRC, f) for f in ("quot_dev.h", "riemann_dev.h", "states_dev.h")]
+DEPS = [SRC] + [os.path.join(CSRC, f) for f in ("quot_dev.h", "riemann_dev.h", "states_dev.h",
+                                                  "adjoint_dev.h")]
 NF = 6000
 
 
@@ -137,3 +138,38 @@ def test_special_values_are_left_to_the_operators(lib, dim):
         assert same[ok].all()
     for gamma in (1.0 + 2.0 ** -12, 80.0):          # outside the ratios Shared takes
         assert not Faces(dim, 6).run(lib, gamma=gamma)[0].any()
+
+
+@pytest.mark.parametrize("scale", [0, 20, 45])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_gradient_reverse_same_bits(lib, dim, scale):
+    """The gradient's reverse with and without Shared quotients: the same bits,
+    for list lengths around its batches, invalid entries, a coincident
+    neighbour and adjoints past the range."""
+    rng = np.random.default_rng(dim + scale)
+    q = dim + 2
+    for trial in range(400):
+        deg = int(rng.integers(1, 12))
+        pow2 = lambda *s: 2.0 ** rng.integers(-scale, scale + 1, s)   # noqa: E731
+        rows = rng.normal(0, 1, (deg, 8)) * pow2(deg, 8)
+        com = rng.normal(0, 1, (deg, 3)) * pow2(deg, 3)
+        area = rng.uniform(0.1, 1.0, deg) * pow2(deg)
+        pv, xi, cx = rng.normal(0, 1, q), rng.normal(0, 1, 3), rng.normal(0, 1, 3)
+        lgrad = rng.normal(0, 1, dim * q)
+        if trial % 5 == 1:
+            area[rng.integers(deg)] = -1.0                  # an invalid entry
+        if trial % 5 == 2:
+            rows[rng.integers(deg), :dim] = xi[:dim]        # no distance
+        if trial % 5 == 3:
+            lgrad[rng.integers(dim * q)] *= 2.0 ** rng.choice([-1000, -310, 320, 900])
+        if trial % 5 == 4:
+            rows[:, dim:dim + q] = pv                       # uniform
+        got = []
+        for fast in (0, 1):
+            lself, lnb = np.ones(q), np.zeros(deg * q)
+            lib.qh_grad_vjp(dim, deg, _p(rows), _p(com), _p(area), _p(pv), _p(xi), _p(cx),
+                            ctypes.c_double(0.7), _p(lgrad), fast, _p(lself), _p(lnb))
+            got.append(np.concatenate([lself, lnb]))
+        a, b = got
+        same = (a.view(np.int64) == b.view(np.int64)) | (np.isnan(a) & np.isnan(b))
+        assert same.all(), (trial, deg, np.nonzero(~same)[0][:4])
