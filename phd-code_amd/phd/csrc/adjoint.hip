@@ -191,7 +191,7 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_face_b(phd_cells c, phd_faces
 // The face list of the cell at sliced position t: entry e's neighbour row from
 // the block's staging (the window's rows, then its halo; from HBM past it) and
 // its face's centroid and area from the slot arrays, coalesced.
-template <int D>
+template <int D, int NQ>
 struct SellNbr {
     int n;
     long long base;                        // slot of entry 0
@@ -201,30 +201,42 @@ struct SellNbr {
     const uint16_t* sloc;
     const double* const* sgeo;
     double* out_rows;                      // the cell's contrib rows
+    int q0;                                // fields q0 .. q0 + NQ - 1
     PHD_HD int deg() const { return n; }
     PHD_HD long long slot(int e) const { return base + (long long)e * 16; }
     PHD_HD bool valid(int e) const { return sloc[slot(e)] != LOC_NONE; }
     PHD_HD void row(int e, double* r) const
     {
         const int loc = sloc[slot(e)];
-        double s[XPW];
-        if (loc != LOC_GLOBAL) {
+        if constexpr (NQ == D + 2) {
+            double s[XPW];
+            if (loc != LOC_GLOBAL) {
 #pragma unroll
-            for (int q = 0; q < XPW / 2; q++) {
-                const double2 v = rows[loc * (XPW / 2) + q];
-                s[2 * q] = v.x;
-                s[2 * q + 1] = v.y;
+                for (int q = 0; q < XPW / 2; q++) {
+                    const double2 v = rows[loc * (XPW / 2) + q];
+                    s[2 * q] = v.x;
+                    s[2 * q + 1] = v.y;
+                }
+            } else {
+                const int j = sj[slot(e)] & 0x7fffffff;
+#pragma unroll
+                for (int q = 0; q < XPW; q++) s[q] = xp[(size_t)j * XPW + q];
             }
+            // as [position | primitive], the order grad_cell_vjp reads
+#pragma unroll
+            for (int k = 0; k < D; k++) r[k] = s[XpLay<D>::X + k];
+#pragma unroll
+            for (int q = 0; q < D + 2; q++) r[D + q] = s[XpLay<D>::P + q];
         } else {
-            const int j = sj[slot(e)] & 0x7fffffff;
+            auto pick = [&](const double* s) {
 #pragma unroll
-            for (int q = 0; q < XPW; q++) s[q] = xp[(size_t)j * XPW + q];
+                for (int k = 0; k < D; k++) r[k] = s[XpLay<D>::X + k];
+#pragma unroll
+                for (int q = 0; q < NQ; q++) r[D + q] = s[XpLay<D>::P + q0 + q];
+            };
+            if (loc != LOC_GLOBAL) pick(reinterpret_cast<const double*>(rows) + loc * XPW);
+            else pick(xp + (size_t)(sj[slot(e)] & 0x7fffffff) * XPW);
         }
-        // as [position | primitive], the order grad_cell_vjp reads
-#pragma unroll
-        for (int k = 0; k < D; k++) r[k] = s[XpLay<D>::X + k];
-#pragma unroll
-        for (int q = 0; q < D + 2; q++) r[D + q] = s[XpLay<D>::P + q];
     }
     PHD_HD void geo(int e, double* cm, double& a) const
     {
@@ -237,67 +249,84 @@ struct SellNbr {
     PHD_HD void out(int e, const double* lam) const
     {
 #pragma unroll
-        for (int q = 0; q < D + 2; q++) out_rows[(size_t)e * (D + 2) + q] = lam[q];
+        for (int q = 0; q < NQ; q++) out_rows[(size_t)e * (D + 2) + q0 + q] = lam[q];
+    }
+};
+
+// The part of a face row's side p that belongs to the fields q0 .. q0 + NQ - 1:
+// their primitives, then their gradients.
+template <int D, int NQ>
+struct RowPart {
+    static constexpr int NF = D + 2, W = NQ * (1 + D);
+    // rows in flight
+    static constexpr int B = NQ < NF ? 8 / NQ : D == 2 ? 3 : 2;
+    double v[W];
+    __device__ __forceinline__ void load(const double* p, int q0)
+    {
+        if constexpr (NQ == NF) {
+#pragma unroll
+            for (int q = 0; q < W / 2; q++) ld2(p + 2 * q, v[2 * q], v[2 * q + 1]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) v[q] = p[q0 + q];
+#pragma unroll
+            for (int q = 0; q < NQ * D; q++) v[NQ + q] = p[NF + q0 * D + q];
+        }
     }
 };
 
 // sum of the face rows of cell cc's list, in list order (the cell's side of
 // each face row)
-template <int D>
-__device__ __forceinline__ void gather_rows(int cc, const int2* __restrict__ csr,
+template <int D, int NQ>
+__device__ __forceinline__ void gather_rows(int cc, int q0, const int2* __restrict__ csr,
                                             const int32_t* __restrict__ off,
                                             const double* __restrict__ frow, double* s)
 {
-    constexpr int PW = pg_width<D>(), W = frow_width<D>();
-    constexpr int B = D == 2 ? 3 : 2;
+    using R = RowPart<D, NQ>;
+    constexpr int PW = pg_width<D>(), W = frow_width<D>(), B = R::B;
     const int beg = off[cc], end = off[cc + 1];
     for (int e0 = beg; e0 < end; e0 += B) {
         int2 en[B];
-        double2 r[B][PW / 2];
+        R r[B];
 #pragma unroll
         for (int b = 0; b < B; b++) en[b] = e0 + b < end ? csr[e0 + b] : make_int2(0, INVALID);
 #pragma unroll
         for (int b = 0; b < B; b++) {
             if ((en[b].y & 0x7fffffff) == INVALID) continue;
-            const double2* p = reinterpret_cast<const double2*>(
-                frow + (size_t)en[b].x * W + ((en[b].y & INCOMING) ? PW : 0));
-#pragma unroll
-            for (int q = 0; q < PW / 2; q++) r[b][q] = p[q];
+            r[b].load(frow + (size_t)en[b].x * W + ((en[b].y & INCOMING) ? PW : 0), q0);
         }
 #pragma unroll
         for (int b = 0; b < B; b++) {
             if ((en[b].y & 0x7fffffff) == INVALID) continue;
 #pragma unroll
-            for (int q = 0; q < PW / 2; q++) { s[2 * q] += r[b][q].x; s[2 * q + 1] += r[b][q].y; }
+            for (int q = 0; q < R::W; q++) s[q] += r[b].v[q];
         }
     }
 }
 
 // The same over the cell's sliced list (face ids coalesced), B rows in flight
-template <int D>
-__device__ __forceinline__ void gather_slots(long long base, int deg,
+template <int D, int NQ>
+__device__ __forceinline__ void gather_slots(long long base, int deg, int q0,
                                              const int32_t* __restrict__ sfi,
                                              const double* __restrict__ frow, double* s)
 {
-    constexpr int PW = pg_width<D>(), W = frow_width<D>(), B = D == 2 ? 3 : 2;
+    using R = RowPart<D, NQ>;
+    constexpr int PW = pg_width<D>(), W = frow_width<D>(), B = R::B;
     for (int e0 = 0; e0 < deg; e0 += B) {
         int en[B];
-        double2 r[B][PW / 2];
+        R r[B];
 #pragma unroll
         for (int b = 0; b < B; b++) en[b] = e0 + b < deg ? sfi[base + (long long)(e0 + b) * 16] : INVALID;
 #pragma unroll
         for (int b = 0; b < B; b++) {
             if (en[b] == INVALID) continue;
-            const double2* p = reinterpret_cast<const double2*>(
-                frow + (size_t)(en[b] & 0x7fffffff) * W + ((en[b] & INCOMING) ? PW : 0));
-#pragma unroll
-            for (int q = 0; q < PW / 2; q++) r[b][q] = p[q];
+            r[b].load(frow + (size_t)(en[b] & 0x7fffffff) * W + ((en[b] & INCOMING) ? PW : 0), q0);
         }
 #pragma unroll
         for (int b = 0; b < B; b++) {
             if (en[b] == INVALID) continue;
 #pragma unroll
-            for (int q = 0; q < PW / 2; q++) { s[2 * q] += r[b][q].x; s[2 * q + 1] += r[b][q].y; }
+            for (int q = 0; q < R::W; q++) s[q] += r[b].v[q];
         }
     }
 }
@@ -312,7 +341,22 @@ __device__ __forceinline__ void gather_slots(long long base, int deg,
 // One block per window, as the gradient kernel, with its staged rows and sliced
 // lists: three walks of the CSR list, each entry two dependent gathers, took 41
 // us at 256^2 and 130 at 21^3, this 38 and 94.
-template <int D>
+//
+// NQ fields a block, blockIdx.y the group: the fields' sums do not meet, so a
+// mesh of few windows is spread over the chip field by field, each block
+// gathering its fields' part of the face rows only.  Such a mesh waits on one
+// block's chain of gathers and of its address unit (80 16-byte loads a cell of
+// 21^3), not on what the chip can do: 8^3 84 -> 46 us, 21^3 94 -> 56, 32^2 24 ->
+// 18, 150^2 38 -> 29.  Where the windows fill the CUs the shared geometry is done
+// NF times over: 28^3 99 us whole and 101 split, 36^3 110 and 240; 200^2 29 and
+// 30, 256^2 40 and 57.
+template <int D> constexpr unsigned adj_split_max() { return D == 2 ? 128 : 80; }
+// blocks of 64 spread the combine's gathers of a small mesh over four times the
+// CUs (21^3 23 -> 15 us with a ghost's entries four at a time, 150^2 7.6 -> 6.3;
+// 1000^2 86 us against 81 with 256)
+constexpr unsigned ADJ_COMBINE_SMALL = 1024;
+
+template <int D, int NQ>
 __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2* __restrict__ csr,
                                                         const int32_t* __restrict__ off,
                                                         const int32_t* __restrict__ perm,
@@ -338,7 +382,8 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2*
                                                         double* __restrict__ lself)
 {
     using Y = Lay<D>;
-    constexpr int NF = Y::NF, PW = pg_width<D>(), HM = halo_max<D>();
+    constexpr int NF = Y::NF, PW = RowPart<D, NQ>::W, HM = halo_max<D>();
+    const int q0 = NQ < NF ? blockIdx.y * NQ : 0;
     __shared__ double2 rows[(PHD_BLOCK + HM) * XPW / 2];
     const long long t = xcd_index(c.n_cells);
     const bool live = t < c.n_cells;
@@ -367,48 +412,45 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2*
     double s[PW];
 #pragma unroll
     for (int q = 0; q < PW; q++) s[q] = 0.0;
-    gather_slots<D>(base, deg, sfi, frow, s);
+    gather_slots<D, NQ>(base, deg, q0, sfi, frow, s);
     for (int a = gofs[i]; a < gofs[i + 1]; a++) {
         const int g = gids[a];
         const int fl = ghost_flips<D>(c, g, reflect, lo, hi);
         double u[PW];
 #pragma unroll
         for (int q = 0; q < PW; q++) u[q] = 0.0;
-        gather_rows<D>(g, csr, off, frow, u);
+        gather_rows<D, NQ>(g, q0, csr, off, frow, u);
 #pragma unroll
-        for (int q = 0; q < D; q++) {
-            if (fl & (1 << q)) {
-                u[1 + q] = -u[1 + q];
-                u[NF + (1 + q) * D + q] = -u[NF + (1 + q) * D + q];
-            }
+        for (int n = 0; n < NQ; n++) {
+            const int q = q0 + n - 1;              // velocity axis of the field
+            if (q < 0 || q >= D || !(fl & (1 << q))) continue;
+            u[n] = -u[n];
+#pragma unroll
+            for (int k = 0; k < D; k++) u[NQ + n * D + k] = k == q ? -u[NQ + n * D + k] : u[NQ + n * D + k];
         }
 #pragma unroll
         for (int q = 0; q < PW; q++) s[q] += u[q];
     }
-    double pv[NF], xi[D], cx[D], own[XPW];
+    double pv[NQ], xi[D], cx[D];
+    const double* own = reinterpret_cast<const double*>(rows) + (i - w0) * XPW;
 #pragma unroll
-    for (int q = 0; q < XPW / 2; q++) {
-        const double2 v = rows[(i - w0) * (XPW / 2) + q];
-        own[2 * q] = v.x;
-        own[2 * q + 1] = v.y;
-    }
-#pragma unroll
-    for (int q = 0; q < NF; q++) pv[q] = own[XpLay<D>::P + q];
+    for (int q = 0; q < NQ; q++) pv[q] = own[XpLay<D>::P + q0 + q];
 #pragma unroll
     for (int k = 0; k < D; k++) { xi[k] = own[XpLay<D>::X + k]; cx[k] = geo[(size_t)i * GEO + k]; }
     const double vol = geo[(size_t)i * GEO + 3];
     const double* const sg[4] = {sx, sy, sz, sa};
-    const SellNbr<D> nb{deg, base, rows, xp, sj, sloc, sg, contrib + (size_t)beg * NF};
+    using Nbr = SellNbr<D, NQ>;
+    const Nbr nb{deg, base, rows, xp, sj, sloc, sg, contrib + (size_t)beg * NF, q0};
     // a row past the staging was not checked
     for (int e = 0; e < deg; e++) fast &= sloc[base + (long long)e * 16] != LOC_GLOBAL;
-    grad_cell_vjp<D>(nb, pv, xi, cx, vol, s + NF, s, fast & within(vol, 0x1p-200, 0x1p100));
+    grad_cell_vjp<D, Nbr, NQ>(nb, pv, xi, cx, vol, s + NQ, s, fast & within(vol, 0x1p-200, 0x1p100));
 #pragma unroll
-    for (int q = 0; q < NF; q++) lself[(size_t)i * NF + q] = s[q];
+    for (int q = 0; q < NQ; q++) lself[(size_t)i * NF + q0 + q] = s[q];
 }
 
 // K3
-template <int D>
-__global__ __launch_bounds__(PHD_BLOCK) void k_adj_combine(phd_cells c, int n_real,
+template <int D, int BS>
+__global__ __launch_bounds__(BS) void k_adj_combine(phd_cells c, int n_real,
                                                            const int32_t* __restrict__ off,
                                                            const int32_t* __restrict__ mirror,
                                                            const int32_t* __restrict__ gofs,
@@ -422,7 +464,7 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_combine(phd_cells c, int n_re
                                                            FaceArrays lam_in)
 {
     constexpr int NF = D + 2, PW = pg_width<D>();
-    long long kk = xcd_index(n_real);
+    long long kk = sched_index<BS, 1>(n_real);
     if (kk >= n_real) return;
     const int k = (int)kk;
     const double lo[3] = {lo0, lo1, lo2}, hi[3] = {hi0, hi1, hi2};
@@ -455,17 +497,28 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_combine(phd_cells c, int n_re
     for (int a = gofs[k]; a < gofs[k + 1]; a++) {
         const int g = gids[a];
         const int fl = ghost_flips<D>(c, g, reflect, lo, hi);
-        for (int e = off[g]; e < off[g + 1]; e++) {
-            const int src = mirror[e];
-            if (src < 0) continue;
-            double t[NF];
+        constexpr int GB = 4;
+        const int gend = off[g + 1];
+        for (int e0 = off[g]; e0 < gend; e0 += GB) {
+            int src[GB];
+            double t[GB][NF];
 #pragma unroll
-            for (int q = 0; q < NF; q++) t[q] = contrib[(size_t)src * NF + q];
+            for (int b = 0; b < GB; b++) src[b] = e0 + b < gend ? mirror[e0 + b] : -1;
 #pragma unroll
-            for (int q = 0; q < D; q++)
-                if (fl & (1 << q)) t[1 + q] = -t[1 + q];
+            for (int b = 0; b < GB; b++) {
+                if (src[b] < 0) continue;
 #pragma unroll
-            for (int q = 0; q < NF; q++) lp[q] += t[q];
+                for (int q = 0; q < NF; q++) t[b][q] = contrib[(size_t)src[b] * NF + q];
+            }
+#pragma unroll
+            for (int b = 0; b < GB; b++) {
+                if (src[b] < 0) continue;
+#pragma unroll
+                for (int q = 0; q < D; q++)
+                    if (fl & (1 << q)) t[b][1 + q] = -t[b][1 + q];
+#pragma unroll
+                for (int q = 0; q < NF; q++) lp[q] += t[b][q];
+            }
         }
     }
     double u[NF], lu[NF];
@@ -516,6 +569,7 @@ int step_vjp(phd_handle* h, phd_plan* p, phd_adjoint* a, const phd_cells* c, con
              double dt, int boost, int gizmo, double* const* lam_out, double* const* lam_in,
              int flags)
 {
+    constexpr int NF = D + 2;
     double l[3] = {0, 0, 0}, u[3] = {0, 0, 0};
     const int refl = boundary == PHD_BOUNDARY_REFLECTIVE;
     if (refl) for (int k = 0; k < D; k++) { l[k] = lo[k]; u[k] = hi[k]; }
@@ -546,13 +600,22 @@ int step_vjp(phd_handle* h, phd_plan* p, phd_adjoint* a, const phd_cells* c, con
         else ADJ_FACES(3);
 #undef ADJ_FACES
     }
-    k_adj_cell<D><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(
-        *c, p->csr, p->off, p->perm, p->sbase, p->sj, p->sfi, p->sgeo[0], p->sgeo[1], p->sgeo[2],
-        p->sgeo[3], p->hcnt, p->halo, p->sloc, p->faces_ok, a->gofs, a->gids, refl, l[0], l[1], l[2], u[0], u[1],
-        u[2], p->xp, p->cell_geo, a->frow, a->contrib, a->lself);
-    k_adj_combine<D><<<xcd_grid(a->n_real), PHD_BLOCK, 0, h->stream>>>(
-        *c, a->n_real, p->off, a->mirror, a->gofs, a->gids, refl, l[0], l[1], l[2], u[0],
-        u[1], u[2], a->lself, a->contrib, gamma, Lo, Li);
+#define ADJ_CELL(NQ)                                                                           \
+    k_adj_cell<D, NQ><<<dim3(xcd_grid(c->n_cells), NF / (NQ)), PHD_BLOCK, 0, h->stream>>>(  \
+        *c, p->csr, p->off, p->perm, p->sbase, p->sj, p->sfi, p->sgeo[0], p->sgeo[1],          \
+        p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc, p->faces_ok, a->gofs, a->gids, refl,\
+        l[0], l[1], l[2], u[0], u[1], u[2], p->xp, p->cell_geo, a->frow, a->contrib, a->lself)
+#define ADJ_COMBINE(BS)                                                                        \
+    k_adj_combine<D, BS><<<sched_grid<BS, 1>(a->n_real), BS, 0, h->stream>>>(                  \
+        *c, a->n_real, p->off, a->mirror, a->gofs, a->gids, refl, l[0], l[1], l[2], u[0],      \
+        u[1], u[2], a->lself, a->contrib, gamma, Lo, Li)
+    const unsigned nw = nblocks(c->n_cells);
+    if (nw < adj_split_max<D>()) ADJ_CELL(1);
+    else ADJ_CELL(NF);
+    if (nw < ADJ_COMBINE_SMALL) ADJ_COMBINE(64);
+    else ADJ_COMBINE(PHD_BLOCK);
+#undef ADJ_CELL
+#undef ADJ_COMBINE
     ADJ_CHK();
     return 0;
 }

@@ -578,12 +578,14 @@ PHD_HD inline void spatial_states_vjp(const double* com, double diff, const doub
 // (cfx -+ dr / 2), with ldf zero or in [2^-300, 2^300]: zero or in [2^-570,
 // 2^510]).  A distance or an ldf outside sends the walk to the operators.  The
 // quotients are 45 of a 3D entry's, and were three quarters of the instructions.
-template <int D, class Nbr>
+//
+// NF fields at a time (all of them, or a part: no field's sums use another's);
+// pv, lgrad, lself, the rows' primitives and out's vector hold these only.
+template <int D, class Nbr, int NF = D + 2>
 PHD_HD inline void grad_cell_vjp(const Nbr& nb, const double* pv, const double* xi,
                                  const double* cx, double vol, const double* lgrad,
                                  double* lself, bool fast = false)
 {
-    constexpr int NF = D + 2;
     const int deg = nb.deg();
     double df[NF * D], pmax[NF], pmin[NF];
     int amax[NF], amin[NF];

@@ -95,3 +95,41 @@ extern "C" void qh_grad_vjp(int dim, int deg, const double* rows, const double* 
     if (dim == 2) grad<2>(deg, rows, com, area, pv, xi, cx, vol, lgrad, fast, lself, lnb);
     else grad<3>(deg, rows, com, area, pv, xi, cx, vol, lgrad, fast, lself, lnb);
 }
+
+namespace {
+
+// the same list with one field of its primitives
+template <int D>
+struct Field : List<D> {
+    int q;
+    void row(int e, double* r) const
+    {
+        for (int k = 0; k < D; k++) r[k] = this->rows[8 * e + k];
+        r[D] = this->rows[8 * e + D + q];
+    }
+    void out(int e, const double* lam) const { this->lnb[(D + 2) * e + q] = lam[0]; }
+};
+
+template <int D>
+void grad_fields(int deg, const double* rows, const double* com, const double* area,
+                 const double* pv, const double* xi, const double* cx, double vol,
+                 const double* lgrad, int fast, double* lself, double* lnb)
+{
+    for (int q = 0; q < D + 2; q++) {
+        Field<D> l;
+        static_cast<List<D>&>(l) = List<D>{deg, rows, com, area, lnb};
+        l.q = q;
+        grad_cell_vjp<D, Field<D>, 1>(l, pv + q, xi, cx, vol, lgrad + q * D, lself + q, fast != 0);
+    }
+}
+
+} // namespace
+
+extern "C" void qh_grad_vjp_fields(int dim, int deg, const double* rows, const double* com,
+                                   const double* area, const double* pv, const double* xi,
+                                   const double* cx, double vol, const double* lgrad, int fast,
+                                   double* lself, double* lnb)
+{
+    if (dim == 2) grad_fields<2>(deg, rows, com, area, pv, xi, cx, vol, lgrad, fast, lself, lnb);
+    else grad_fields<3>(deg, rows, com, area, pv, xi, cx, vol, lgrad, fast, lself, lnb);
+}

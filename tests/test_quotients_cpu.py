@@ -143,8 +143,9 @@ def test_special_values_are_left_to_the_operators(lib, dim):
 @pytest.mark.parametrize("scale", [0, 20, 45])
 @pytest.mark.parametrize("dim", [2, 3])
 def test_gradient_reverse_same_bits(lib, dim, scale):
-    """The gradient's reverse with and without Shared quotients: the same bits,
-    for list lengths around its batches, invalid entries, a coincident
+    """The gradient's reverse with and without Shared quotients, all fields at
+    once and one by one: the same bits, for list lengths around its batches,
+    invalid entries, a coincident
     neighbour and adjoints past the range."""
     rng = np.random.default_rng(dim + scale)
     q = dim + 2
@@ -165,11 +166,13 @@ def test_gradient_reverse_same_bits(lib, dim, scale):
         if trial % 5 == 4:
             rows[:, dim:dim + q] = pv                       # uniform
         got = []
-        for fast in (0, 1):
+        for vjp, fast in ((lib.qh_grad_vjp, 0), (lib.qh_grad_vjp, 1),
+                          (lib.qh_grad_vjp_fields, 0), (lib.qh_grad_vjp_fields, 1)):
             lself, lnb = np.ones(q), np.zeros(deg * q)
-            lib.qh_grad_vjp(dim, deg, _p(rows), _p(com), _p(area), _p(pv), _p(xi), _p(cx),
-                            ctypes.c_double(0.7), _p(lgrad), fast, _p(lself), _p(lnb))
+            vjp(dim, deg, _p(rows), _p(com), _p(area), _p(pv), _p(xi), _p(cx),
+                ctypes.c_double(0.7), _p(lgrad), fast, _p(lself), _p(lnb))
             got.append(np.concatenate([lself, lnb]))
-        a, b = got
-        same = (a.view(np.int64) == b.view(np.int64)) | (np.isnan(a) & np.isnan(b))
-        assert same.all(), (trial, deg, np.nonzero(~same)[0][:4])
+        a = got[0]
+        for b in got[1:]:
+            same = (a.view(np.int64) == b.view(np.int64)) | (np.isnan(a) & np.isnan(b))
+            assert same.all(), (trial, deg, np.nonzero(~same)[0][:4])
