@@ -552,7 +552,11 @@ __device__ __forceinline__ void load_row(const double* xp, int j, double* r)
 // dphi: two divisions per field instead of one per face, same bits.
 //
 // Registers: 2D is held to 128 (4 waves per SIMD, no spills; it would take 129).
-template <int D, int LIM, int BS = PHD_BLOCK, int XCD = 1>
+//
+// NQ fields a block, blockIdx.y the group (AREPO: the fields' sums and limiters do
+// not meet); four entries in flight, as one field's rows are short.  The first
+// group writes the record's centroid.
+template <int D, int LIM, int BS = PHD_BLOCK, int XCD = 1, int NQ = D + 2>
 __global__ __launch_bounds__(BS)
 __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cells, const int8_t* __restrict__ tag,
                                                          const double* __restrict__ geo,
@@ -573,7 +577,9 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                                                          double* __restrict__ rec, int ld)
 {
     using Y = Lay<D>;
-    constexpr int NF = Y::NF;
+    constexpr bool SPLIT = NQ < Y::NF;             // fields q0 .. q0 + NQ - 1 only
+    static_assert(!SPLIT || (BS == SORT_WINDOW && LIM == PHD_LIMITER_AREPO));
+    const int q0 = SPLIT ? blockIdx.y * NQ : 0;
     // A block of SORT_WINDOW threads owns one whole window of cells (the
     // degree sort permutes within windows): every thread stages its cell's
     // packed row in LDS, and the block then gathers the window's halo (the
@@ -596,7 +602,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
     // one stream (a lane storing its own record touches a line per 16 bytes:
     // 421 -> 367 us on the 256-problem ensemble).  In 3D the values held past
     // the barrier cost a wave per SIMD or spill (573 us, 688 or 579).
-    constexpr bool STREAM = STAGE && D == 2;
+    constexpr bool STREAM = STAGE && D == 2 && !SPLIT;
     constexpr int Q = Y::LD / 2;
     constexpr int NROWS = (SORT_WINDOW + HM) * XPW / 2, NCACHE = KC * SORT_WINDOW;
     constexpr int NOUT = STREAM ? SORT_WINDOW * Q : 0;
@@ -641,7 +647,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
     if (!STREAM && !real) return;
     double out[Y::LD];
     if (real) {
-        double cx[D], vol, xi[D], pv[NF];
+        double cx[D], vol, xi[D], pv[NQ];
         {
             if (D == 2) {
                 // the packed row's centroid pair and the dense volume array: 24
@@ -660,10 +666,15 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
 #pragma unroll
             for (int k = 0; k < D; k++) xi[k] = own[XpLay<D>::X + k];
 #pragma unroll
-            for (int n = 0; n < NF; n++) pv[n] = own[XpLay<D>::P + n];
+            for (int n = 0; n < NQ; n++) {
+                if constexpr (SPLIT)
+                    pv[n] = reinterpret_cast<const double*>(rows)[(i - w0) * XPW + XpLay<D>::P + q0 + n];
+                else
+                    pv[n] = own[XpLay<D>::P + n];
+            }
         }
         fast &= within(vol, 0x1p-200, 0x1p100);
-        double pmax[NF], pmin[NF], df[NF * D];
+        double pmax[NQ], pmin[NQ], df[NQ * D];
         const int deg = off[i + 1] - off[i];
         const long long base = sbase[t / SLICE] + (t % SLICE);
         // The sums over the list, in the arithmetic ar; false when a row that was
@@ -674,7 +685,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
             constexpr bool SHARED = std::decay_t<decltype(ar)>::fast;
             bool ok = true;
 #pragma unroll
-            for (int n = 0; n < NF; n++) {
+            for (int n = 0; n < NQ; n++) {
                 pmax[n] = pmin[n] = pv[n];
 #pragma unroll
                 for (int k = 0; k < D; k++) df[n * D + k] = 0.0;
@@ -682,10 +693,18 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
             // GB entries in flight: their slot loads, then their row reads, then the
             // entries applied one by one in list order (the same sums).  128^3: one
             // 625 us, two 573, three 737 (2 waves per SIMD); 2D ensemble: 484, 421, 463.
-            constexpr int GB = 2;
+            constexpr int GB = SPLIT ? 4 : 2;
+            // a row in registers: whole, or [position | the block's fields]
+            constexpr int RX = SPLIT ? 0 : XpLay<D>::X, RP = SPLIT ? D : XpLay<D>::P;
             for (int e0 = 0; e0 < deg; e0 += GB) {
                 SlotEnt<D> cur[GB];
-                double rb[GB][XPW];
+                double rb[GB][SPLIT ? D + NQ : XPW];
+                auto pick = [&](double* r, const double* s) {
+#pragma unroll
+                    for (int k = 0; k < D; k++) r[k] = s[XpLay<D>::X + k];
+#pragma unroll
+                    for (int n = 0; n < NQ; n++) r[D + n] = s[XpLay<D>::P + q0 + n];
+                };
 #pragma unroll
                 for (int b = 0; b < GB; b++) {
                     cur[b].j = INVALID;
@@ -715,16 +734,28 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                     const long long lj = (long long)j - w0;
                     if (HALO ? j != LOC_GLOBAL : (STAGE && lj >= 0 && lj < SORT_WINDOW)) {
                         const double2* row = rows + (HALO ? (long long)j : lj) * (XPW / 2);
+                        if constexpr (SPLIT) {
+                            pick(rb[b], reinterpret_cast<const double*>(row));
+                        } else {
 #pragma unroll
-                        for (int q = 0; q < XPW / 2; q++) {
-                            const double2 v = row[q];
-                            rb[b][2 * q] = v.x;
-                            rb[b][2 * q + 1] = v.y;
+                            for (int q = 0; q < XPW / 2; q++) {
+                                const double2 v = row[q];
+                                rb[b][2 * q] = v.x;
+                                rb[b][2 * q + 1] = v.y;
+                            }
                         }
                     } else {
                         const long long slot = base + (long long)(e0 + b) * SLICE;
-                        load_row(xp, HALO ? sj[slot] & 0x7fffffff : j, rb[b]);
-                        if (SHARED) ok &= row_ok<D>(rb[b]);
+                        const int jg = HALO ? sj[slot] & 0x7fffffff : j;
+                        double r[XPW];
+                        load_row(xp, jg, r);
+                        if (SHARED) ok &= row_ok<D>(r);
+                        if constexpr (SPLIT) {
+                            pick(rb[b], xp + (size_t)jg * XPW);
+                        } else {
+#pragma unroll
+                            for (int q = 0; q < XPW; q++) rb[b][q] = r[q];
+                        }
                     }
                 }
 #pragma unroll
@@ -736,7 +767,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                     double cfx[D], dr[D], rr = 0.0;
 #pragma unroll
                     for (int k = 0; k < D; k++) {
-                        const double xj = r[XpLay<D>::X + k];
+                        const double xj = r[RX + k];
                         cfx[k] = com[k] - 0.5 * (xi[k] + xj);
                         dr[k] = xi[k] - xj;
                         rr += dr[k] * dr[k];
@@ -745,8 +776,8 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                     // Springel (2010) eq. 21 summand, area*(...)/(r*vol) (677-681)
                     const auto rv = ar.rcp(ar.root(rr) * vol);
 #pragma unroll
-                    for (int n = 0; n < NF; n++) {
-                        const double pj = r[XpLay<D>::P + n];
+                    for (int n = 0; n < NQ; n++) {
+                        const double pj = r[RP + n];
                         pmax[n] = fmax(pmax[n], pj);
                         pmin[n] = fmin(pmin[n], pj);
                         const double d_dif = pj - pv[n];
@@ -764,13 +795,13 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
         // face centroids in flight in the limiter pass (two measured best)
         constexpr int LB = 2;
 
-        double alpha[NF];
+        double alpha[NQ];
 #pragma unroll
-        for (int n = 0; n < NF; n++) alpha[n] = 1.0;
+        for (int n = 0; n < NQ; n++) alpha[n] = 1.0;
         if (LIM == PHD_LIMITER_AREPO) {
-            double dpos[NF], dneg[NF];
+            double dpos[NQ], dneg[NQ];
 #pragma unroll
-            for (int n = 0; n < NF; n++) { dpos[n] = 0.0; dneg[n] = 0.0; }
+            for (int n = 0; n < NQ; n++) { dpos[n] = 0.0; dneg[n] = 0.0; }
             for (int e0 = 0; e0 < deg; e0 += LB) {
                 double relb[LB][D];
 #pragma unroll
@@ -791,7 +822,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                 for (int b = 0; b < LB; b++) {
                     if (e0 + b >= deg) continue;
 #pragma unroll
-                    for (int n = 0; n < NF; n++) {
+                    for (int n = 0; n < NQ; n++) {
                         double dphi = 0.0;
 #pragma unroll
                         for (int k = 0; k < D; k++) dphi += df[n * D + k] * relb[b][k];
@@ -806,7 +837,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                 }
             }
 #pragma unroll
-            for (int n = 0; n < NF; n++) {
+            for (int n = 0; n < NQ; n++) {
                 if (dpos[n] > 0) alpha[n] = fmin(alpha[n], fmax((pmax[n] - pv[n]) / dpos[n], 0.));
                 if (dneg[n] < 0) alpha[n] = fmin(alpha[n], fmax((pmin[n] - pv[n]) / dneg[n], 0.));
             }
@@ -839,7 +870,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                     load_row(xp, j, r);
                 }
 #pragma unroll
-                for (int n = 0; n < NF; n++) {
+                for (int n = 0; n < NQ; n++) {
                     double dphi = 0.0;
 #pragma unroll
                     for (int k = 0; k < D; k++) dphi += df[n * D + k] * (cm[k] - cx[k]);
@@ -854,10 +885,25 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                 }
             }
         }
+        if constexpr (SPLIT) {
+            double* const o = rec + (size_t)i * ld;
 #pragma unroll
-        for (int n = 0; n < NF; n++) out[Y::P0 + n] = pv[n];
+            for (int n = 0; n < NQ; n++) {
+                o[Y::P0 + q0 + n] = pv[n];
 #pragma unroll
-        for (int n = 0; n < NF; n++)
+                for (int k = 0; k < D; k++) o[Y::G0 + (q0 + n) * D + k] = alpha[n] * df[n * D + k];
+            }
+            if (q0 == 0) {
+#pragma unroll
+                for (int k = 0; k < D; k++) o[Y::C0 + k] = cx[k];
+                if (Y::LD > Y::REC) o[Y::LD - 1] = 0.0;
+            }
+            return;
+        }
+#pragma unroll
+        for (int n = 0; n < NQ; n++) out[Y::P0 + n] = pv[n];
+#pragma unroll
+        for (int n = 0; n < NQ; n++)
 #pragma unroll
             for (int k = 0; k < D; k++) out[Y::G0 + n * D + k] = alpha[n] * df[n * D + k];
 #pragma unroll
@@ -1676,6 +1722,14 @@ int launch_pack(phd_handle* h, phd_plan* p, const phd_cells* c)
     return 0;
 }
 
+// Windows below which the gradients are formed field by field (NQ = 1): such a
+// mesh leaves CUs idle, and its time is one wave's chain of entries, which is
+// shorter with one field's sums (8^3 22.7 -> 16.2 us, 21^3 29.0 -> 23.4, 32^2 11.4
+// -> 8.3, 100^2 13.1 -> 9.9).  From there on the geometry that the fields share
+// is done NF times over: 112 windows in 3D 31.6 and 30.3 us, 216 32.5 and 56.1;
+// in 2D 136 windows 14.2 and 13.7 us, 200 14.7 and 16.7.
+template <int D> constexpr int grad_split_max() { return D == 2 ? 128 : 100; }
+
 template <int D>
 int launch_grad(phd_handle* h, phd_plan* p, const phd_cells* c, int limiter, double* rec, int ld)
 {
@@ -1685,9 +1739,16 @@ int launch_grad(phd_handle* h, phd_plan* p, const phd_cells* c, int limiter, dou
         LAUNCHCHK();
     }
     const unsigned nb = xcd_grid(c->n_cells);
-#define GS(L) k_grad_sell<D, L><<<nb, PHD_BLOCK, 0, h->stream>>>(c->n_cells, c->tag, p->cell_geo, c->volume, p->xp, p->off, p->perm, p->sbase, p->sj, p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc, p->faces_ok, rec, ld)
-    if (limiter == PHD_LIMITER_AREPO) GS(PHD_LIMITER_AREPO);
-    else if (limiter == PHD_LIMITER_TESS) GS(PHD_LIMITER_TESS);
+    constexpr int NF = D + 2;
+#define GS(L, NQ)                                                                              \
+    k_grad_sell<D, L, PHD_BLOCK, 1, NQ><<<dim3(nb, NF / (NQ)), PHD_BLOCK, 0, h->stream>>>(     \
+        c->n_cells, c->tag, p->cell_geo, c->volume, p->xp, p->off, p->perm, p->sbase, p->sj,   \
+        p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc,             \
+        p->faces_ok, rec, ld)
+    if (limiter == PHD_LIMITER_AREPO) {
+        if (n_windows(c) < grad_split_max<D>()) GS(PHD_LIMITER_AREPO, 1);
+        else GS(PHD_LIMITER_AREPO, NF);
+    } else if (limiter == PHD_LIMITER_TESS) GS(PHD_LIMITER_TESS, NF);
     else return PHD_E_MODE;
 #undef GS
     LAUNCHCHK();
