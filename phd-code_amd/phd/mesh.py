@@ -143,9 +143,12 @@ class Mesh(object):
                             geometry=not self.device_geometry)
         ng = geo["ghost_map"].size
         dev = particles.device
-        if ng and "map" in particles.carrays and dev.type == "cuda":
+        groups = particles.carray_named_groups
+        if ng and "map" in particles.carrays and dev.type == "cuda" \
+                and "primitive" in groups and "conservative" in groups:
             # room for the ghosts, then one pass over all fields takes them
-            # from their images (extract and append are two calls per field)
+            # from their images (extract and append are two calls per field);
+            # the pass reads the cells through a view of these groups
             particles.extend(ng)
             particles["tag"][n:] = ParticleTAGS.Ghost
             particles["map"][n:] = torch.as_tensor(geo["ghost_map"], device=dev)
