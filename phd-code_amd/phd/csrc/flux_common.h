@@ -58,7 +58,7 @@ struct phd_plan {
                                  // follows all its incoming faces (faces in owner order)
     int32_t* ghosts;             // third allocation: the ghost cells (tag 1), ascending
     int n_ghosts;
-    // fourth allocation (3D): each window's halo, the first halo_max of the
+    // fourth allocation: each window's halo, the first halo_max of the
     // distinct cells outside the window that its real cells' lists name
     // (ascending, halo[w * halo_max + k] for k < hcnt[w]), and per slot the
     // row of the gradient kernel's LDS staging that holds the neighbour
@@ -81,9 +81,9 @@ constexpr int INVALID = 0x7fffffff;
 constexpr int FREC = 8;      // doubles per face record, at most
 constexpr uint16_t LOC_GLOBAL = 0xFFFE, LOC_NONE = 0xFFFF;   // sloc markers
 // halo rows the gradient kernel stages beside its window's 256 rows: 576 in
-// 3D (53 KB of LDS per block, three blocks per CU as its registers allow);
-// none in 2D, where a tenth of the entries lie outside the window and the
-// staging code would cost the kernel its fourth wave per SIMD
+// 3D (53 KB of LDS per block, three blocks per CU as its registers allow), 112
+// in 2D, where a tenth of the entries lie outside the window (40 KB with the
+// cached centroids, four blocks per CU)
 template <int D> constexpr int halo_max() { return D == 2 ? 112 : 576; }
 
 // Face record: com(D) | area | normal(D) | |x_j - x_i|, 6 doubles in 2D and

@@ -25,10 +25,9 @@
 // square root), so the results are bit-identical to it.
 //
 // The 3D face kernel makes three passes over the face's vertices (vertex
-// mean, fan about the mean, tetrahedra about the face centroid) and
-// recomputes each circumcentre per pass instead of holding a variable-length
-// vertex list: the ring entries and generator rows it re-reads stay in L1/L2,
-// and the extra arithmetic is cheaper than per-lane scratch arrays.
+// mean, fan about the mean, tetrahedra about the face centroid).  A face whose
+// ring is staged keeps its vertices in LDS over the ring's positions; the few
+// past the staging recompute each circumcentre per pass.
 #include <stdlib.h>
 #include "flux_common.h"
 

@@ -376,7 +376,7 @@ __device__ __forceinline__ int block_scan_excl(int v, int* part, int& total)
     return ex;
 }
 
-// The 3D gradient kernel's halo of window w (cells [w0, w1) = positions
+// The gradient kernels' halo of window w (cells [w0, w1) = positions
 // [w0, w1), since the degree sort permutes within windows), one block per
 // window: the list entries of its real cells that name a cell outside the
 // window are gathered into LDS, sorted (bitonic) and made distinct; the
@@ -1935,7 +1935,7 @@ int build_slots(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces*
     return rc;
 }
 
-// Per window of SORT_WINDOW cells, the halo the 3D gradient kernel stages
+// Per window of SORT_WINDOW cells, the halo the gradient kernels stage
 // in LDS beside the window's own rows (at most halo_max rows, fixed stride
 // per window), and each slot's row in that staging: k_plan_halo, one block
 // per window, after the sliced lists are built.
