@@ -14,6 +14,19 @@ from . import _native as nat
 from .views import cells_view
 
 
+def copy_from_images(particles, fields):
+    """Every ghost takes the listed fields from its image, on the GPU.  Only
+    tag and map are read beside them: the container's groups play no part."""
+    lib, h = nat.flux(), nat.handle()
+    c = nat.Cells()
+    c.dim, c.n_cells = len(particles.carray_named_groups["position"]), particles.get_carray_size()
+    c.tag, c.map = particles.pointer("tag"), particles.pointer("map")
+    ptrs = (ctypes.c_void_p * len(fields))(*[particles.pointer(f) for f in fields])
+    size = (ctypes.c_int32 * len(fields))(*[particles.carrays[f].element_size() for f in fields])
+    nat.check(lib.phd_update_ghost_fields(h, ctypes.byref(c), ptrs, size, len(fields)),
+              "update_ghost_fields")
+
+
 class BoundaryConditionBase(object):
     native_code = None
 

@@ -20,6 +20,7 @@ import torch
 
 from . import _native as nat
 from .containers import CarrayContainer
+from .domain import copy_from_images
 from .utils import ParticleTAGS
 from .views import cells_view, faces_view
 
@@ -71,6 +72,17 @@ def face_lists_from_pairs(pair_i, pair_j, n_cells):
     off = np.zeros(n_cells + 1, dtype=np.int32)
     np.cumsum(counts, out=off[1:])
     return off, fids[order].astype(np.int32)
+
+
+def _copied_on_gpu(particles):
+    """Whether the kernel that copies ghosts from their images can take this
+    container: int8 tags, an int32 map, and arrays of the container's capacity
+    that it can address by element, on the device the library works on."""
+    a, dev, whole = particles.carrays, particles.device, (particles._cap,)
+    return (dev.type == "cuda" and dev.index in (None, torch.cuda.current_device())
+            and "map" in a and a["map"].dtype == torch.int32 and a["tag"].dtype == torch.int8
+            and all(t.shape == whole and t.is_contiguous() and t.element_size() in (1, 4, 8)
+                    for t in a.values()))
 
 
 class Mesh(object):
@@ -143,17 +155,13 @@ class Mesh(object):
                             geometry=not self.device_geometry)
         ng = geo["ghost_map"].size
         dev = particles.device
-        groups = particles.carray_named_groups
-        if ng and "map" in particles.carrays and dev.type == "cuda" \
-                and "primitive" in groups and "conservative" in groups:
+        if ng and _copied_on_gpu(particles):
             # room for the ghosts, then one pass over all fields takes them
-            # from their images (extract and append are two calls per field);
-            # the pass reads the cells through a view of these groups
+            # from their images (extract and append are two calls per field)
             particles.extend(ng)
             particles["tag"][n:] = ParticleTAGS.Ghost
             particles["map"][n:] = torch.as_tensor(geo["ghost_map"], device=dev)
-            domain_manager.update_ghost_fields(
-                particles, [f for f in particles.carrays if f not in ("tag", "map")])
+            copy_from_images(particles, [f for f in particles.carrays if f not in ("tag", "map")])
             particles["type"][n:] = ParticleTAGS.Exterior
             if not self.device_geometry:
                 for k, f in enumerate(particles.carray_named_groups["position"]):
