@@ -108,24 +108,29 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_prim_from_cons(phd_cells c, doubl
 // one per 256 cells took 102 us at 128^3 (the 53 MB read take 9).  So at most
 // CFL_BLOCKS blocks of 1024 threads, one a CU, walk the cells: 27 us there (the
 // pow of each cell's radius bounds it now), and 14.8 -> 6.9 us at 512^2 in 2D.
+// Up to cfl_small cells blocks of 256 threads cost fewer atomics than the 1024
+// threads' pows and final step on fewer CUs: 1.7 k cells in 3D 3.5 and 4.6 us, 24 k
+// 4.0 and 5.9, 55 k 5.0 and 5.9, 74 k 5.8 and 5.8; 2D 10 k 3.2 and 4.2, 23 k 3.5 and
+// 4.1, 41 k 4.4 and 4.2, 67 k 5.6 and 4.4.
 constexpr int CFL_THREADS = 1024, CFL_BLOCKS = 256;
+template <int D> constexpr int cfl_small() { return D == 2 ? 32768 : 65536; }
 
-template <int D>
-__global__ __launch_bounds__(CFL_THREADS) void k_cfl(phd_cells c, double gamma, int boost,
-                                                     unsigned long long* err)
+template <int D, int BS>
+__global__ __launch_bounds__(BS) void k_cfl(phd_cells c, double gamma, int boost,
+                                            unsigned long long* err)
 {
     double v = __longlong_as_double((long long)INF_BITS);
-    for (long long i = (long long)blockIdx.x * CFL_THREADS + threadIdx.x; i < c.n_cells;
-         i += (long long)gridDim.x * CFL_THREADS)
+    for (long long i = (long long)blockIdx.x * BS + threadIdx.x; i < c.n_cells;
+         i += (long long)gridDim.x * BS)
         if (c.tag[i] == 0) v = fmin(v, cfl_value<D>(c, i, gamma, boost));
     for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-    __shared__ double wmin[CFL_THREADS / 64];
+    __shared__ double wmin[BS / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0) wmin[wid] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         double b = wmin[0];
-        for (int w = 1; w < CFL_THREADS / 64; w++) b = fmin(b, wmin[w]);
+        for (int w = 1; w < BS / 64; w++) b = fmin(b, wmin[w]);
         atomicMin(&err[3], (unsigned long long)__double_as_longlong(b));
     }
 }
@@ -1820,6 +1825,16 @@ int launch_face(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces*
     return PHD_E_MODE;
 }
 
+template <int D>
+void launch_cfl(phd_handle* h, const phd_cells* c, double gamma, int boost)
+{
+    if (c->n_cells <= cfl_small<D>())
+        k_cfl<D, PHD_BLOCK><<<nblocks(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, gamma, boost, h->d_err);
+    else
+        k_cfl<D, CFL_THREADS><<<std::min((c->n_cells - 1) / CFL_THREADS + 1, CFL_BLOCKS), CFL_THREADS, 0,
+                                h->stream>>>(*c, gamma, boost, h->d_err);
+}
+
 // A 3D cell's rows are 80 uncoalesced loads, and the waves of one block share a
 // CU's address unit: a mesh of few blocks is updated by 64-thread blocks, which
 // spread over four times the CUs (21^3 14.5 -> 11.5 us, 41^3 22.8 -> 20.4; 2D,
@@ -2179,9 +2194,8 @@ int phd_compute_time_step(phd_handle* h, const phd_cells* c, double gamma, doubl
     if (!h || check_cells(c) || !dt_out || c->n_cells == 0) return PHD_E_ARG;
     k_reset_err<<<1, 64, 0, h->stream>>>(h->d_err);   // also clears the fault words
     LAUNCHCHK();
-    const int nb = std::min((c->n_cells - 1) / CFL_THREADS + 1, CFL_BLOCKS);
-    if (c->dim == 2) k_cfl<2><<<nb, CFL_THREADS, 0, h->stream>>>(*c, gamma, boost, h->d_err);
-    else k_cfl<3><<<nb, CFL_THREADS, 0, h->stream>>>(*c, gamma, boost, h->d_err);
+    if (c->dim == 2) launch_cfl<2>(h, c, gamma, boost);
+    else launch_cfl<3>(h, c, gamma, boost);
     LAUNCHCHK();
     HIPCHK(hipMemcpyAsync(h->h_err + 3, h->d_err + 3, sizeof(unsigned long long), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
