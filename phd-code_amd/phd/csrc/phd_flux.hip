@@ -1308,19 +1308,54 @@ __global__ __launch_bounds__(BS) void k_update_sell(phd_cells c, const double* _
     update_body<D, BS, XCD, OR>(c, RowSummands{g}, csr, off, perm, sbase, sfi, cinfo, err);
 }
 
-// The update from the caller's flux arrays and areas.  A face gathered from them
-// costs D + 3 cache lines, so the block first forms the summands of its
-// window's owned faces (one id range when the faces are in owner order) in LDS,
-// from coalesced loads, and both cells' entries read them there; the rest are
-// gathered.  CAP rows leave two blocks a CU their LDS in 3D (about 2020 faces a
-// window) and five in 2D (768).  Against a walk of the CSR entries one by one:
-// 512^2 in 2D 41 -> 28 us, 41^3 54 -> 39 us.
-// Fewer windows than flux_stage_min leave CUs idle, and the staging is then one
-// more latency of the few blocks there are (staged and not: 150^2 11.2 and 8.1 us,
-// 256^2 14.4 and 12.5, 400^2 16.6 and 18.8; 30^3 32 and 28, 41^3 38 and 50); in 3D
-// 64-thread blocks then spread the gathers over more CUs (21^3 26 -> 20 us).
-template <int D> constexpr int flux_stage_min() { return D == 2 ? 512 : 256; }
+// The update from the caller's flux arrays and areas, three ways.
+//
+// Small meshes (below flux_stage_min windows) walk each cell's list entry by
+// entry, k_update: their time is the chain perm -> slot -> face of the sliced
+// lists, and the CSR has one link less; blocks of 64 spread the cells over more
+// CUs (walk / sliced lists: 100^2 6.1 / 7.7 us, 256^2 9.3 / 12.2, 21^3 16.6 / 19.9,
+// 32^3 23.9 / 29.3; in 256-thread blocks 7.8, 11.8, 22.4 and 25.8).
+//
+// Larger ones, faces in owner order: a face gathered from the arrays costs D + 3
+// cache lines, so the block first forms the summands of its window's owned faces
+// (one id range) in LDS, from coalesced loads, and both cells' entries read them
+// there; the rest are gathered.  flux_cap rows and the update's own staging leave
+// four blocks a CU their LDS in 2D (800 rows; a window owns about 768 faces) and
+// two in 3D (1750 of about 2020).  Walk / staged: 400^2 15.8 / 16.7 us, 450^2 20.9 /
+// 17.9, 512^2 38.2 / 27.4; 36^3 30.0 / 32.2, 40^3 48.4 / 36.4, 48^3 137 / 42.
+//
+// Larger ones with faces in any other order take the sliced lists, whose
+// entries load coalesced (walk / sliced, cells renumbered at random: 450^2 105 /
+// 101 us, 800^2 381 / 341, 40^3 119 / 105, 64^3 599 / 489; below the line 256^2 22.5
+// / 25.2, 21^3 16.1 / 19.7).
+template <int D> constexpr int flux_stage_min() { return D == 2 ? 700 : 256; }
 template <int D> constexpr int flux_cap() { return D == 2 ? 800 : 1750; }
+
+template <int D>
+__global__ __launch_bounds__(64) void k_update(phd_cells c, FluxSummands src,
+                                               const int2* __restrict__ csr,
+                                               const int32_t* __restrict__ off,
+                                               unsigned long long* err)
+{
+    constexpr int NF = D + 2;
+    const long long ii = sched_index<64, 1>(c.n_cells);
+    if (ii >= c.n_cells) return;
+    const int i = (int)ii;
+    const int beg = off[i], end = off[i + 1];
+    if (ghost_fault<D>(c, i, beg, end, csr, err)) return;
+    double u[NF];
+#pragma unroll
+    for (int q = 0; q < NF; q++) u[q] = c.cons[q][i];
+    for (int e = beg; e < end; e++) {
+        const int2 en = csr[e];
+        if ((en.y & 0x7fffffff) == INVALID) continue;
+        double s[NF];
+        src.template get<D>(en.x, s);
+        if (apply_summand<D>(u, s, en.y & INCOMING, en.x, err)) break;
+    }
+#pragma unroll
+    for (int q = 0; q < NF; q++) c.cons[q][i] = u[q];
+}
 
 struct StagedSummands {
     FluxSummands far;
@@ -1338,9 +1373,9 @@ struct StagedSummands {
     }
 };
 
-template <int D, int OR, int STAGED, int BS>
-__global__ __launch_bounds__(BS) void k_update_flux(phd_cells c, int n_faces,
-                                                           FluxSummands src,
+// OR: the faces are in owner order, and the window's are staged
+template <int D, int OR>
+__global__ __launch_bounds__(PHD_BLOCK) void k_update_flux(phd_cells c, int n_faces, FluxSummands src,
                                                            const int2* __restrict__ csr,
                                                            const int32_t* __restrict__ off,
                                                            const int32_t* __restrict__ perm,
@@ -1349,7 +1384,7 @@ __global__ __launch_bounds__(BS) void k_update_flux(phd_cells c, int n_faces,
                                                            const int2* __restrict__ cinfo,
                                                            unsigned long long* err)
 {
-    if constexpr (STAGED) {
+    if constexpr (OR) {
         __shared__ double rows[flux_cap<D>() * (D + 2)];
         __shared__ int first;
         const long long t = xcd_index(c.n_cells);
@@ -1368,10 +1403,10 @@ __global__ __launch_bounds__(BS) void k_update_flux(phd_cells c, int n_faces,
             for (int q = 0; q < D + 2; q++) rows[k * (D + 2) + q] = s[q];
         }
         __syncthreads();
-        update_body<D, PHD_BLOCK, 1, OR>(c, StagedSummands{src, rows, f0, n}, csr, off, perm, sbase,
-                                         sfi, cinfo, err);
+        update_body<D, PHD_BLOCK, 1, 1>(c, StagedSummands{src, rows, f0, n}, csr, off, perm, sbase,
+                                        sfi, cinfo, err);
     } else {
-        update_body<D, BS, 1, OR>(c, src, csr, off, perm, sbase, sfi, cinfo, err);
+        update_body<D, PHD_BLOCK, 1, 0>(c, src, csr, off, perm, sbase, sfi, cinfo, err);
     }
 }
 
@@ -1858,11 +1893,11 @@ template <int D>
 int launch_update_flux(phd_handle* h, phd_plan* p, const phd_cells* c, const FluxSummands& src)
 {
     if (c->n_cells == 0) return 0;
-#define UF(OR, ST, BS) k_update_flux<D, OR, ST, BS><<<sched_grid<BS, 1>(c->n_cells), BS, 0, h->stream>>>(*c, p->n_faces, src, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
-    if (!p->owner_runs) UF(0, 0, PHD_BLOCK);
-    else if (n_windows(c) >= flux_stage_min<D>()) UF(1, 1, PHD_BLOCK);
-    else if (D == 3) UF(1, 0, 64);
-    else UF(1, 0, PHD_BLOCK);
+#define UF(OR) k_update_flux<D, OR><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, p->n_faces, src, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
+    if (n_windows(c) < flux_stage_min<D>())
+        k_update<D><<<sched_grid<64, 1>(c->n_cells), 64, 0, h->stream>>>(*c, src, p->csr, p->off, h->d_err);
+    else if (p->owner_runs) UF(1);
+    else UF(0);
 #undef UF
     LAUNCHCHK();
     return 0;
