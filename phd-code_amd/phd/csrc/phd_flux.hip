@@ -1874,15 +1874,16 @@ void launch_cfl(phd_handle* h, const phd_cells* c, double gamma, int boost)
 // CU's address unit: a mesh of few blocks is updated by 64-thread blocks, which
 // spread over four times the CUs (21^3 14.5 -> 11.5 us, 41^3 22.8 -> 20.4; 2D,
 // with a fifth of the loads, gains nothing).
-template <int D> constexpr int small_update() { return D == 3 ? 512 : 0; }
+constexpr int SMALL_UPDATE = 512;
 
 template <int D>
 int launch_update(phd_handle* h, phd_plan* p, const phd_cells* c)
 {
     if (c->n_cells == 0) return 0;
+    constexpr int SMALL = D == 3 ? 64 : PHD_BLOCK;
 #define UB(OR, BS) k_update_sell<D, BS, 1, OR><<<sched_grid<BS, 1>(c->n_cells), BS, 0, h->stream>>>(*c, p->g, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
     if (!p->owner_runs) UB(0, PHD_BLOCK);
-    else if (n_windows(c) < small_update<D>()) UB(1, 64);
+    else if (n_windows(c) < SMALL_UPDATE) UB(1, SMALL);
     else UB(1, PHD_BLOCK);
 #undef UB
     LAUNCHCHK();
