@@ -17,6 +17,8 @@ assert _CELLS.size == nat.ctypes.sizeof(nat.Cells) and _FACES.size == nat.ctypes
 
 def _ptrs(arrays, names, room):
     p = [arrays[f].data_ptr() for f in names]
+    if len(p) > room:
+        raise IndexError("a group of %d fields where the view holds %d" % (len(p), room))
     return p + [0] * (room - len(p))
 
 
