@@ -220,20 +220,32 @@ def flux():
     return _flux if _flux is not None else load_flux_library()
 
 
+def _current_stream(dev):
+    return torch.cuda.current_stream(dev).cuda_stream
+
+
+# the same number without the Stream object around it (0.1 us instead of 1.1, some
+# ten times a step), in versions of torch that have it
+_current_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _current_stream)
+
+
 def handle(device=None):
     """Per-device library handle, with its stream set to torch's current one."""
     lib = flux()
-    dev = torch._C._cuda_getDevice() if device is None else int(device)
+    if device is None:
+        dev = torch.cuda.current_device()
+    else:
+        torch.cuda.init()                 # either refuses in a forked child
+        dev = int(device)
     h = _handles.get(dev)
     if h is None:
-        torch.cuda.init()
         hp = c_vp()
         rc = lib.phd_handle_create(ctypes.byref(hp), dev)
         if rc != 0:
             raise RuntimeError("phd_handle_create failed: %s" % lib.phd_error_string(rc).decode())
         h = hp.value
         _handles[dev] = h
-    lib.phd_set_stream(h, torch._C._cuda_getCurrentRawStream(dev))
+    lib.phd_set_stream(h, _current_stream(dev))
     return h
 
 
