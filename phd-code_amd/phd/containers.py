@@ -107,8 +107,9 @@ class CarrayContainer(object):
         if moved == 0:
             self._size = n
             return
+        at = keep.nonzero().squeeze(1)       # once for all arrays
         for name, t in self.carrays.items():
-            t[:n] = t[:self._size][keep]
+            t[:n] = t[:self._size][at]
         self._size = n
 
     def extract_items(self, indices, fields=None):
