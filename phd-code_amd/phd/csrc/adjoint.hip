@@ -443,7 +443,7 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2*
     const Nbr nb{deg, base, rows, xp, sj, sloc, sg, contrib + (size_t)beg * NF, q0};
     // a row past the staging was not checked
     for (int e = 0; e < deg; e++) fast &= sloc[base + (long long)e * 16] != LOC_GLOBAL;
-    grad_cell_vjp<D, Nbr, NQ>(nb, pv, xi, cx, vol, s + NQ, s, fast & within(vol, 0x1p-200, 0x1p100));
+    grad_cell_vjp<D, Nbr, NQ>(nb, pv, xi, cx, vol, s + NQ, s, fast & vol_ok(vol));
 #pragma unroll
     for (int q = 0; q < NQ; q++) lself[(size_t)i * NF + q0 + q] = s[q];
 }

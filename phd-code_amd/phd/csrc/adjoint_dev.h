@@ -572,12 +572,12 @@ PHD_HD inline void spatial_states_vjp(const double* com, double diff, const doub
 // the neighbour's primitives through out(e, lam).
 //
 // fast: every position, primitive, face centroid and area of the list and the
-// cell's own is zero or in [2^-100, 2^100] and vol in [2^-200, 2^100], so that
-// the quotients by r * vol may be taken with Shared (the ranges are worked out
-// at the gradient kernel's; in the second walk the numerators are ldf * area *
-// (cfx -+ dr / 2), with ldf zero or in [2^-300, 2^300]: zero or in [2^-570,
-// 2^510]).  A distance or an ldf outside sends the walk to the operators.  The
-// quotients are 45 of a 3D entry's, and were three quarters of the instructions.
+// cell's own and vol are in the ranges of quot_dev.h, so that the quotients by
+// r * vol may be taken with Shared.  (In the second walk the numerators are ldf *
+// area * (cfx -+ dr / 2), with ldf zero or in [2^-300, 2^300]: zero or in [2^-653,
+// 2^553], their quotients in [2^-905, 2^906].)  A distance or an ldf outside sends
+// the walk to the operators.  The quotients are 45 of a 3D entry's, and were three
+// quarters of the instructions.
 //
 // NF fields at a time (all of them, or a part: no field's sums use another's);
 // pv, lgrad, lself, the rows' primitives and out's vector hold these only.

@@ -53,7 +53,7 @@ struct phd_plan {
     int2* cinfo;                 // per position: incoming count, first owned face
     double* sgeo[4];             // face centroid x, y, z, area per slot
     double* g;                   // per-face update summand rows (dt*area)*flux, F x GW
-    int faces_ok;                // every face centroid and area is zero or in [2^-100, 2^100]
+    int faces_ok;                // every face's centroid and area are in the ranges of quot_dev.h
     int owner_runs;              // every real cell's owned faces are one id run that
                                  // follows all its incoming faces (faces in owner order)
     int32_t* ghosts;             // third allocation: the ghost cells (tag 1), ascending
@@ -228,31 +228,18 @@ __device__ __forceinline__ void ld2(const double* p, double& a, double& b)
     b = v.y;
 }
 
-// x == 0 or |x| in [2^-100, 2^100]; false for inf and NaN (non-short-circuit
-// operators: the test compiles to compares and mask logic, no branches)
-__device__ __forceinline__ bool operand_ok(double x)
-{
-    const double ax = fabs(x);
-    return (ax <= 0x1p100) & ((ax >= 0x1p-100) | (x == 0.0));
-}
-
-// Ranges of the gradient sums' operands, for the Shared arithmetic (quot_dev.h).
-// With every position, primitive, face centroid and area zero or in [2^-100,
-// 2^100] and volumes in [2^-200, 2^100]: differences and sums of them are zero
-// or >= 2^-153, the distance r = sqrt(sum dr^2) lies in [2^-153, 2^102] unless
-// zero, r * vol in [2^-353, 2^202], and the numerators area * (...) are zero or
-// in [2^-459, 2^304].  So the values are checked once, where a row is staged and
-// (the faces) where the plan is made, and not the numerators of every entry.
-//
-// row_ok: every value of a packed row that the gradients take
+// Every value of a packed row that the gradient sums take is in the range of
+// the Shared arithmetic (quot_dev.h).  The values are checked once, where a row is
+// staged and (the faces) where the plan is made, and not the numerators of every
+// entry.
 template <int D>
 __device__ __forceinline__ bool row_ok(const double* r)
 {
     bool ok = true;
 #pragma unroll
-    for (int k = 0; k < D; k++) ok &= operand_ok(r[XpLay<D>::X + k]);
+    for (int k = 0; k < D; k++) ok &= coord_ok(r[XpLay<D>::X + k]);
 #pragma unroll
-    for (int n = 0; n < D + 2; n++) ok &= operand_ok(r[XpLay<D>::P + n]);
+    for (int n = 0; n < D + 2; n++) ok &= prim_ok(r[XpLay<D>::P + n]);
     return ok;
 }
 

@@ -208,9 +208,9 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_plan_faces(phd_cells c, phd_faces
         diff += dx * dx;          // reconstruction.pyx:866
     }
     r[F::A] = f.area[m];
-    bool ok = operand_ok(r[F::A]);
+    bool ok = area_ok(r[F::A]);
 #pragma unroll
-    for (int k = 0; k < D; k++) ok &= operand_ok(r[F::C + k]);
+    for (int k = 0; k < D; k++) ok &= coord_ok(r[F::C + k]);
     if (!ok) atomicMin(flag, 0ull);
     r[F::DIFF] = sqrt(diff);      // reconstruction.pyx:875
     double2* o = reinterpret_cast<double2*>(rec + (size_t)m * F::W);
@@ -678,7 +678,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
                     pv[n] = own[XpLay<D>::P + n];
             }
         }
-        fast &= within(vol, 0x1p-200, 0x1p100);
+        fast &= vol_ok(vol);
         double pmax[NQ], pmin[NQ], df[NQ * D];
         const int deg = off[i + 1] - off[i];
         const long long base = sbase[t / SLICE] + (t % SLICE);
