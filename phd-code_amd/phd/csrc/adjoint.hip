@@ -190,8 +190,9 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_face_b(phd_cells c, phd_faces
 
 // The face list of the cell at sliced position t: entry e's neighbour row from
 // the block's staging (the window's rows, then its halo; from HBM past it) and
-// its face's centroid and area from the slot arrays, coalesced.
-template <int D, int NQ>
+// its face's centroid and area from the slot arrays, coalesced.  HL: the plan
+// keeps its windows' halos; without them the window's rows are found by id.
+template <int D, int NQ, int HL>
 struct SellNbr {
     int n;
     long long base;                        // slot of entry 0
@@ -202,12 +203,20 @@ struct SellNbr {
     const double* const* sgeo;
     double* out_rows;                      // the cell's contrib rows
     int q0;                                // fields q0 .. q0 + NQ - 1
+    int w0;                                // the window's first cell
     PHD_HD int deg() const { return n; }
     PHD_HD long long slot(int e) const { return base + (long long)e * 16; }
-    PHD_HD bool valid(int e) const { return sloc[slot(e)] != LOC_NONE; }
+    PHD_HD int place(int e) const
+    {
+        if constexpr (HL) return sloc[slot(e)];
+        const int j = sj[slot(e)] & 0x7fffffff;
+        const unsigned k = (unsigned)(j - w0);
+        return j == INVALID ? LOC_NONE : k < PHD_BLOCK ? (int)k : LOC_GLOBAL;
+    }
+    PHD_HD bool valid(int e) const { return place(e) != LOC_NONE; }
     PHD_HD void row(int e, double* r) const
     {
-        const int loc = sloc[slot(e)];
+        const int loc = place(e);
         if constexpr (NQ == D + 2) {
             double s[XPW];
             if (loc != LOC_GLOBAL) {
@@ -356,7 +365,7 @@ template <int D> constexpr unsigned adj_split_max() { return D == 2 ? 128 : 80; 
 // 1000^2 86 us against 81 with 256)
 constexpr unsigned ADJ_COMBINE_SMALL = 1024;
 
-template <int D, int NQ>
+template <int D, int NQ, int HL>
 __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2* __restrict__ csr,
                                                         const int32_t* __restrict__ off,
                                                         const int32_t* __restrict__ perm,
@@ -382,7 +391,7 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2*
                                                         double* __restrict__ lself)
 {
     using Y = Lay<D>;
-    constexpr int NF = Y::NF, PW = RowPart<D, NQ>::W, HM = halo_max<D>();
+    constexpr int NF = Y::NF, PW = RowPart<D, NQ>::W, HM = HL ? halo_max<D>() : 0;
     const int q0 = NQ < NF ? blockIdx.y * NQ : 0;
     __shared__ double2 rows[(PHD_BLOCK + HM) * XPW / 2];
     const long long t = xcd_index(c.n_cells);
@@ -399,7 +408,7 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2*
         for (int q = 0; q < XPW / 2; q++) rows[at * (XPW / 2) + q] = make_double2(r[2 * q], r[2 * q + 1]);
     };
     if (live) stage(t, threadIdx.x);
-    if (w0 < c.n_cells) {
+    if (HL && w0 < c.n_cells) {
         const long long w = w0 / PHD_BLOCK;
         const int hn = hcnt[w];
         for (int k = threadIdx.x; k < hn; k += PHD_BLOCK) stage(halo[w * HM + k], PHD_BLOCK + k);
@@ -439,10 +448,10 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_adj_cell(phd_cells c, const int2*
     for (int k = 0; k < D; k++) { xi[k] = own[XpLay<D>::X + k]; cx[k] = geo[(size_t)i * GEO + k]; }
     const double vol = geo[(size_t)i * GEO + 3];
     const double* const sg[4] = {sx, sy, sz, sa};
-    using Nbr = SellNbr<D, NQ>;
-    const Nbr nb{deg, base, rows, xp, sj, sloc, sg, contrib + (size_t)beg * NF, q0};
+    using Nbr = SellNbr<D, NQ, HL>;
+    const Nbr nb{deg, base, rows, xp, sj, sloc, sg, contrib + (size_t)beg * NF, q0, (int)w0};
     // a row past the staging was not checked
-    for (int e = 0; e < deg; e++) fast &= sloc[base + (long long)e * 16] != LOC_GLOBAL;
+    for (int e = 0; e < deg; e++) fast &= nb.place(e) != LOC_GLOBAL;
     grad_cell_vjp<D, Nbr, NQ>(nb, pv, xi, cx, vol, s + NQ, s, fast & vol_ok(vol));
 #pragma unroll
     for (int q = 0; q < NQ; q++) lself[(size_t)i * NF + q0 + q] = s[q];
@@ -600,8 +609,12 @@ int step_vjp(phd_handle* h, phd_plan* p, phd_adjoint* a, const phd_cells* c, con
         else ADJ_FACES(3);
 #undef ADJ_FACES
     }
+    constexpr int NO_HALO = D == 3;                // 3D plans always keep halos
 #define ADJ_CELL(NQ)                                                                           \
-    k_adj_cell<D, NQ><<<dim3(xcd_grid(c->n_cells), NF / (NQ)), PHD_BLOCK, 0, h->stream>>>(  \
+    if (p->sloc) ADJ_CELL_H(NQ, 1);                                                            \
+    else ADJ_CELL_H(NQ, NO_HALO)
+#define ADJ_CELL_H(NQ, HL)                                                                     \
+    k_adj_cell<D, NQ, HL><<<dim3(xcd_grid(c->n_cells), NF / (NQ)), PHD_BLOCK, 0, h->stream>>>(  \
         *c, p->csr, p->off, p->perm, p->sbase, p->sj, p->sfi, p->sgeo[0], p->sgeo[1],          \
         p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc, p->faces_ok, a->gofs, a->gids, refl,\
         l[0], l[1], l[2], u[0], u[1], u[2], p->xp, p->cell_geo, a->frow, a->contrib, a->lself)
@@ -610,11 +623,12 @@ int step_vjp(phd_handle* h, phd_plan* p, phd_adjoint* a, const phd_cells* c, con
         *c, a->n_real, p->off, a->mirror, a->gofs, a->gids, refl, l[0], l[1], l[2], u[0],      \
         u[1], u[2], a->lself, a->contrib, gamma, Lo, Li)
     const unsigned nw = nblocks(c->n_cells);
-    if (nw < adj_split_max<D>()) ADJ_CELL(1);
-    else ADJ_CELL(NF);
+    if (nw < adj_split_max<D>()) { ADJ_CELL(1); }
+    else { ADJ_CELL(NF); }
     if (nw < ADJ_COMBINE_SMALL) ADJ_COMBINE(64);
     else ADJ_COMBINE(PHD_BLOCK);
 #undef ADJ_CELL
+#undef ADJ_CELL_H
 #undef ADJ_COMBINE
     ADJ_CHK();
     return 0;

@@ -63,7 +63,8 @@ struct phd_plan {
     // (ascending, halo[w * halo_max + k] for k < hcnt[w]), and per slot the
     // row of the gradient kernel's LDS staging that holds the neighbour
     // (sloc: window rows 0..255, then halo rows; LOC_GLOBAL past the
-    // staging, LOC_NONE for an invalid neighbour)
+    // staging, LOC_NONE for an invalid neighbour).  Null in a 2D plan of
+    // scattered cells.
     void* halo_base;
     int32_t* hcnt;
     int32_t* halo;

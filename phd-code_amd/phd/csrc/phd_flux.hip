@@ -286,6 +286,31 @@ constexpr int SORT_WINDOW = PHD_BLOCK;   // cells per degree-sorted window
 
 inline long long n_windows(const phd_cells* c) { return ((long long)c->n_cells + SORT_WINDOW - 1) / SORT_WINDOW; }
 
+// 2D: whether the window's halo is worth staging.  Up to HALO_SAMPLE windows,
+// spread evenly, add up 4 * (entries of their real cells that leave the window) -
+// entries: positive where cells are numbered row by row or at random.  A halo then
+// holds several times the rows that are staged, and staging some of them made the
+// gradients of such meshes slower than gathering all (256^2 by rows 23.3 and 20.8 us,
+// at random 29.2 and 27.4; along a curve, a tenth of the entries, 19.2 and 21.0).
+constexpr int HALO_SAMPLE = 64;
+
+__global__ __launch_bounds__(SORT_WINDOW) void k_plan_outside(phd_cells c, const int2* csr,
+                                                              const int32_t* off, int n_windows,
+                                                              unsigned long long* sum)
+{
+    const long long w0 = (long long)blockIdx.x * n_windows / gridDim.x * SORT_WINDOW;
+    const long long i = w0 + threadIdx.x;
+    int v = 0;
+    if (i < c.n_cells && c.tag[i] == 0) {
+        for (int e = off[i]; e < off[i + 1]; e++) {
+            const int o = csr[e].y & 0x7fffffff;
+            v += o != INVALID && (o < w0 || o >= w0 + SORT_WINDOW) ? 3 : -1;
+        }
+    }
+    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(sum, (unsigned long long)(long long)v);
+}
+
 // width of each 16-cell slice = the largest face-list length of its real cells
 // position -> cell order: inside each window of SORT_WINDOW consecutive
 // cells, real cells by descending face count (ties by id), then ghosts
@@ -561,7 +586,9 @@ __device__ __forceinline__ void load_row(const double* xp, int j, double* r)
 // NQ fields a block, blockIdx.y the group (AREPO: the fields' sums and limiters do
 // not meet); four entries in flight, as one field's rows are short.  The first
 // group writes the record's centroid.
-template <int D, int LIM, int BS = PHD_BLOCK, int XCD = 1, int NQ = D + 2>
+//
+// HL: the plan keeps its windows' halos (phd_plan::sloc).
+template <int D, int LIM, int BS, int XCD, int NQ, int HL>
 __global__ __launch_bounds__(BS)
 __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cells, const int8_t* __restrict__ tag,
                                                          const double* __restrict__ geo,
@@ -594,7 +621,7 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
     // per-lane HBM gather (about 1/4 of the entries in 3D, 1/10 in 2D
     // lie outside the window; a wave would wait for its slowest lane).
     constexpr bool STAGE = BS == SORT_WINDOW;
-    constexpr int HM = STAGE ? halo_max<D>() : 0;
+    constexpr int HM = STAGE && HL ? halo_max<D>() : 0;
     constexpr bool HALO = HM > 0;
     // 2D AREPO: the first KC entries of each list keep their face centroid
     // in LDS from the gradient pass for the limiter pass ([entry][thread],
@@ -1780,17 +1807,22 @@ int launch_grad(phd_handle* h, phd_plan* p, const phd_cells* c, int limiter, dou
     }
     const unsigned nb = xcd_grid(c->n_cells);
     constexpr int NF = D + 2;
+    constexpr int NO_HALO = D == 3;                // 3D plans always keep halos
 #define GS(L, NQ)                                                                              \
-    k_grad_sell<D, L, PHD_BLOCK, 1, NQ><<<dim3(nb, NF / (NQ)), PHD_BLOCK, 0, h->stream>>>(     \
+    if (p->sloc) GSH(L, NQ, 1);                                                                \
+    else GSH(L, NQ, NO_HALO)
+#define GSH(L, NQ, HL)                                                                         \
+    k_grad_sell<D, L, PHD_BLOCK, 1, NQ, HL><<<dim3(nb, NF / (NQ)), PHD_BLOCK, 0, h->stream>>>( \
         c->n_cells, c->tag, p->cell_geo, c->volume, p->xp, p->off, p->perm, p->sbase, p->sj,   \
         p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc,             \
         p->faces_ok, rec, ld)
     if (limiter == PHD_LIMITER_AREPO) {
-        if (n_windows(c) < grad_split_max<D>()) GS(PHD_LIMITER_AREPO, 1);
-        else GS(PHD_LIMITER_AREPO, NF);
-    } else if (limiter == PHD_LIMITER_TESS) GS(PHD_LIMITER_TESS, NF);
+        if (n_windows(c) < grad_split_max<D>()) { GS(PHD_LIMITER_AREPO, 1); }
+        else { GS(PHD_LIMITER_AREPO, NF); }
+    } else if (limiter == PHD_LIMITER_TESS) { GS(PHD_LIMITER_TESS, NF); }
     else return PHD_E_MODE;
 #undef GS
+#undef GSH
     LAUNCHCHK();
     return 0;
 }
@@ -1989,15 +2021,16 @@ int build_slots(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces*
 // Per window of SORT_WINDOW cells, the halo the gradient kernels stage
 // in LDS beside the window's own rows (at most halo_max rows, fixed stride
 // per window), and each slot's row in that staging: k_plan_halo, one block
-// per window, after the sliced lists are built.
-int build_halo(phd_handle* h, phd_plan* p, const phd_cells* c)
+// per window, after the sliced lists are built.  A 2D plan of scattered cells
+// keeps none.
+int build_halo(phd_handle* h, phd_plan* p, const phd_cells* c, bool scattered)
 {
     const long long na = c->n_cells, nw = (na + SORT_WINDOW - 1) / SORT_WINDOW;
     const long long nsl = p->n_slots;
     const int HM = c->dim == 2 ? halo_max<2>() : halo_max<3>();
     p->hcnt = p->halo = nullptr;
     p->sloc = nullptr;
-    if (HM == 0) return 0;            // no halo staging in this dimension
+    if (c->dim == 2 && scattered) return 0;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t s_hc = al(4 * (size_t)nw + 4), s_ha = al(4 * (size_t)nw * HM + 4);
     const size_t s_sl = al(2 * (size_t)nsl + 2);
@@ -2165,16 +2198,18 @@ int phd_plan_create(phd_handle* h, const phd_cells* c, const phd_faces* f, phd_p
             else k_plan_cells<3><<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, p->cell_geo, p->xp);
             k_plan_csr<<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->csr, p->d_bad);
             k_plan_runs<<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, p->csr, p->off, p->d_bad + 1);
+            const int nw = (int)n_windows(c);
+            if (D == 2) k_plan_outside<<<std::min(nw, HALO_SAMPLE), SORT_WINDOW, 0, h->stream>>>(*c, p->csr, p->off, nw, p->d_bad + 3);
         }
         if (hipPeekAtLastError() != hipSuccess) { (void)hipGetLastError(); rc = PHD_E_HIP; break; }
-        unsigned long long bad[3] = {NOERR, NOERR, NOERR};
+        unsigned long long bad[4] = {NOERR, NOERR, NOERR, INF_BITS};
         if (hipMemcpyAsync(bad, p->d_bad, sizeof(bad), hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
             hipStreamSynchronize(h->stream) != hipSuccess) { rc = PHD_E_HIP; break; }
         p->bad_cell = bad[0] == NOERR ? -1 : (long long)bad[0];
         p->owner_runs = bad[1] == NOERR;
         p->faces_ok = bad[2] == NOERR;
         rc = build_slots(h, p, c, f);
-        if (!rc) rc = build_halo(h, p, c);
+        if (!rc) rc = build_halo(h, p, c, (long long)(bad[3] - INF_BITS) > 0);   // slot 3 starts there
         if (!rc) rc = build_ghost_list(h, p, c);
     } while (0);
     if (rc) {
@@ -2571,17 +2606,23 @@ int batch_grad(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_schedul
         LAUNCHCHK();
     }
     const long long n = c->n_cells;
-#define X(BS, XC)                                                                              \
-    if (s.grad_block == BS && s.xcd == XC) {                                                   \
-        k_grad_sell<D, PHD_LIMITER_AREPO, BS, XC><<<sched_grid<BS, XC>(n), BS, 0, h->stream>>>( \
+#define GB(BS, XC, HL)                                                                         \
+    k_grad_sell<D, PHD_LIMITER_AREPO, BS, XC, D + 2, HL>                                       \
+        <<<sched_grid<BS, XC>(n), BS, 0, h->stream>>>(                                         \
             c->n_cells, c->tag, p->cell_geo, c->volume, p->xp, p->off, p->perm, p->sbase,      \
             p->sj, p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->hcnt, p->halo, p->sloc,  \
-            p->faces_ok, rec, ld);                                                                          \
+            p->faces_ok, rec, ld)
+#define X(BS, XC)                                                                              \
+    if (s.grad_block == BS && s.xcd == XC) {                                                   \
+        constexpr int NO_HALO = D == 3 || BS != SORT_WINDOW;   /* the same instance */         \
+        if (p->sloc) GB(BS, XC, 1);                                                            \
+        else GB(BS, XC, NO_HALO);                                                              \
         LAUNCHCHK();                                                                           \
         return 0;                                                                              \
     }
     PHD_SCHED_CASES(X)
 #undef X
+#undef GB
     return PHD_E_ARG;
 }
 
