@@ -235,25 +235,42 @@ __global__ __launch_bounds__(PHD_BLOCK) void k_plan_cells(phd_cells c, double* g
 }
 
 // per entry {face id, other cell | incoming bit}; the neighbor check of
-// reconstruction.pyx:647-652 is evaluated here once per mesh
+// reconstruction.pyx:647-652 is evaluated here once per mesh (bad[0]).
+//
+// Of every `every`-th window (0: none) bad[3] adds up 4 * (entries of its real
+// cells that leave the window) - entries.  The sum is positive where cells are
+// numbered row by row or at random.  The halo of such a 2D window holds several
+// times the rows that are staged, and staging some of them made the gradients
+// slower than gathering all (256^2 by rows 23.3 and 20.8 us, at random 29.2 and
+// 27.4; along a curve, where a tenth of the entries leave, 19.2 and 21.0).
+constexpr int HALO_SAMPLE = 64;
+
 __global__ __launch_bounds__(PHD_BLOCK) void k_plan_csr(phd_cells c, phd_faces f, int2* csr,
-                                                        unsigned long long* bad)
+                                                        unsigned long long* bad, int every)
 {
-    long long i = xcd_index(c.n_cells);
-    if (i >= c.n_cells) return;
-    const int beg = f.nbr_off[i], end = f.nbr_off[i + 1];
-    for (int e = beg; e < end; e++) {
-        int fid = f.nbr_face[e];
-        int a = f.pair_i[fid], b = f.pair_j[fid];
-        int other;
-        if (a == (int)i) other = b;
-        else if (b == (int)i) other = a | INCOMING;
-        else {
-            other = INVALID;
-            if (c.tag[i] == 0) atomicMin(bad, (unsigned long long)i);
+    const long long i = xcd_index(c.n_cells), w0 = i - threadIdx.x;
+    int leave = 0;
+    if (i < c.n_cells) {
+        const int beg = f.nbr_off[i], end = f.nbr_off[i + 1];
+        const bool real = c.tag[i] == 0;
+        for (int e = beg; e < end; e++) {
+            int fid = f.nbr_face[e];
+            int a = f.pair_i[fid], b = f.pair_j[fid];
+            int other;
+            if (a == (int)i) other = b;
+            else if (b == (int)i) other = a | INCOMING;
+            else {
+                other = INVALID;
+                if (real) atomicMin(bad, (unsigned long long)i);
+            }
+            csr[e] = make_int2(fid, other);
+            const int o = other & 0x7fffffff;
+            if (real) leave += o != INVALID && (o < w0 || o >= w0 + PHD_BLOCK) ? 3 : -1;
         }
-        csr[e] = make_int2(fid, other);
     }
+    if (every == 0 || (w0 / PHD_BLOCK) % every != 0) return;      // block-uniform
+    for (int d = 32; d > 0; d >>= 1) leave += __shfl_xor(leave, d, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(bad + 3, (unsigned long long)(long long)leave);
 }
 
 // owner_runs check: in every real cell's list, the owned faces (not
@@ -285,31 +302,6 @@ constexpr int SLICE = 16;
 constexpr int SORT_WINDOW = PHD_BLOCK;   // cells per degree-sorted window
 
 inline long long n_windows(const phd_cells* c) { return ((long long)c->n_cells + SORT_WINDOW - 1) / SORT_WINDOW; }
-
-// 2D: whether the window's halo is worth staging.  Up to HALO_SAMPLE windows,
-// spread evenly, add up 4 * (entries of their real cells that leave the window) -
-// entries: positive where cells are numbered row by row or at random.  A halo then
-// holds several times the rows that are staged, and staging some of them made the
-// gradients of such meshes slower than gathering all (256^2 by rows 23.3 and 20.8 us,
-// at random 29.2 and 27.4; along a curve, a tenth of the entries, 19.2 and 21.0).
-constexpr int HALO_SAMPLE = 64;
-
-__global__ __launch_bounds__(SORT_WINDOW) void k_plan_outside(phd_cells c, const int2* csr,
-                                                              const int32_t* off, int n_windows,
-                                                              unsigned long long* sum)
-{
-    const long long w0 = (long long)blockIdx.x * n_windows / gridDim.x * SORT_WINDOW;
-    const long long i = w0 + threadIdx.x;
-    int v = 0;
-    if (i < c.n_cells && c.tag[i] == 0) {
-        for (int e = off[i]; e < off[i + 1]; e++) {
-            const int o = csr[e].y & 0x7fffffff;
-            v += o != INVALID && (o < w0 || o >= w0 + SORT_WINDOW) ? 3 : -1;
-        }
-    }
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(sum, (unsigned long long)(long long)v);
-}
 
 // width of each 16-cell slice = the largest face-list length of its real cells
 // position -> cell order: inside each window of SORT_WINDOW consecutive
@@ -1936,8 +1928,6 @@ int launch_update_flux(phd_handle* h, phd_plan* p, const phd_cells* c, const Flu
     return 0;
 }
 
-// sliced face lists of a plan: widths on the device, bases by a host prefix
-// sum (plan creation is the synchronising, allocating call), then the slots
 // the ghost cells (tag 1) in ascending order, for the kernels that touch
 // ghosts only
 int build_ghost_list(phd_handle* h, phd_plan* p, const phd_cells* c)
@@ -1959,15 +1949,16 @@ int build_ghost_list(phd_handle* h, phd_plan* p, const phd_cells* c)
     return 0;
 }
 
-int build_slots(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces* f)
+// sliced face lists of a plan: widths on the device (in d_w), bases by a host
+// prefix sum (plan creation is the synchronising, allocating call), then the
+// slots
+int build_slots(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces* f, int32_t* d_w)
 {
     const long long na = c->n_cells, nf = f->n_faces;
     const int D = c->dim, NF = D + 2;
     const long long ns = (na + SLICE - 1) / SLICE;
-    int32_t* d_w = nullptr;
-    HIPCHK(hipMalloc(&d_w, sizeof(int32_t) * (size_t)(ns + 1)));
     int32_t* hw = (int32_t*)malloc(sizeof(int32_t) * (size_t)(ns + 1));
-    if (!hw) { (void)hipFree(d_w); return PHD_E_ARG; }
+    if (!hw) return PHD_E_ARG;
     int rc = 0;
     long long total = 0;
     do {
@@ -1984,7 +1975,6 @@ int build_slots(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces*
         hw[ns] = (int32_t)total;
         if (total >= INT32_MAX) { rc = PHD_E_ARG; break; }
     } while (0);
-    (void)hipFree(d_w);
     if (rc) { free(hw); return rc; }
     p->n_slots = total;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -2005,8 +1995,8 @@ int build_slots(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces*
     p->cinfo = (int2*)b;
     do {
         if (hipMemcpyAsync(p->sbase, hw, sizeof(int32_t) * (size_t)(ns + 1), hipMemcpyHostToDevice, h->stream) != hipSuccess) { rc = PHD_E_HIP; break; }
-        if (total > 0) k_fill_i32<<<nblocks(total), PHD_BLOCK, 0, h->stream>>>(p->sj, total, INVALID);
-        if (total > 0) k_fill_i32<<<nblocks(total), PHD_BLOCK, 0, h->stream>>>(p->sfi, total, INVALID);
+        const long long nfill = (long long)(2 * s_j / sizeof(int32_t));   // sj, then sfi
+        if (total > 0) k_fill_i32<<<nblocks(nfill), PHD_BLOCK, 0, h->stream>>>(p->sj, nfill, INVALID);
         if (na > 0) {
             if (D == 2) k_plan_slots<2><<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->csr, p->off, p->perm, p->sbase, p->sj, p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->sfi, p->cinfo);
             else k_plan_slots<3><<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->csr, p->off, p->perm, p->sbase, p->sj, p->sgeo[0], p->sgeo[1], p->sgeo[2], p->sgeo[3], p->sfi, p->cinfo);
@@ -2025,7 +2015,7 @@ int build_slots(phd_handle* h, phd_plan* p, const phd_cells* c, const phd_faces*
 // keeps none.
 int build_halo(phd_handle* h, phd_plan* p, const phd_cells* c, bool scattered)
 {
-    const long long na = c->n_cells, nw = (na + SORT_WINDOW - 1) / SORT_WINDOW;
+    const long long na = c->n_cells, nw = n_windows(c);
     const long long nsl = p->n_slots;
     const int HM = c->dim == 2 ? halo_max<2>() : halo_max<3>();
     p->hcnt = p->halo = nullptr;
@@ -2163,7 +2153,8 @@ int phd_plan_create(phd_handle* h, const phd_cells* c, const phd_faces* f, phd_p
     const size_t s_xp = al(sizeof(double) * XPW * (size_t)na);
     const size_t s_perm = al(sizeof(int32_t) * (size_t)na);
     const size_t s_bad = al(4 * sizeof(unsigned long long));
-    const size_t total = s_face + s_geo + s_csr + s_off + s_xp + s_perm + s_bad;
+    const size_t s_w = al(sizeof(int32_t) * (size_t)(na / SLICE + 2));   // slice widths
+    const size_t total = s_face + s_geo + s_csr + s_off + s_xp + s_perm + s_bad + s_w;
     phd_plan* p = new phd_plan();
     p->dim = D;
     p->n_cells = (int)na;
@@ -2180,7 +2171,8 @@ int phd_plan_create(phd_handle* h, const phd_cells* c, const phd_faces* f, phd_p
     p->off = (int32_t*)b; b += s_off;
     p->xp = (double*)b; b += s_xp;
     p->perm = (int32_t*)b; b += s_perm;
-    p->d_bad = (unsigned long long*)b;
+    p->d_bad = (unsigned long long*)b; b += s_bad;
+    int32_t* const widths = (int32_t*)b;
     p->slot_base = nullptr;
     p->ghosts = nullptr;
     p->n_ghosts = 0;
@@ -2194,12 +2186,11 @@ int phd_plan_create(phd_handle* h, const phd_cells* c, const phd_faces* f, phd_p
             else k_plan_faces<3><<<xcd_grid(nf), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->face_rec, p->d_bad + 2);
         }
         if (na > 0) {
+            const int every = D == 2 ? (int)(n_windows(c) / HALO_SAMPLE) + 1 : 0;
             if (D == 2) k_plan_cells<2><<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, p->cell_geo, p->xp);
             else k_plan_cells<3><<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, p->cell_geo, p->xp);
-            k_plan_csr<<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->csr, p->d_bad);
+            k_plan_csr<<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, *f, p->csr, p->d_bad, every);
             k_plan_runs<<<xcd_grid(na), PHD_BLOCK, 0, h->stream>>>(*c, p->csr, p->off, p->d_bad + 1);
-            const int nw = (int)n_windows(c);
-            if (D == 2) k_plan_outside<<<std::min(nw, HALO_SAMPLE), SORT_WINDOW, 0, h->stream>>>(*c, p->csr, p->off, nw, p->d_bad + 3);
         }
         if (hipPeekAtLastError() != hipSuccess) { (void)hipGetLastError(); rc = PHD_E_HIP; break; }
         unsigned long long bad[4] = {NOERR, NOERR, NOERR, INF_BITS};
@@ -2208,8 +2199,9 @@ int phd_plan_create(phd_handle* h, const phd_cells* c, const phd_faces* f, phd_p
         p->bad_cell = bad[0] == NOERR ? -1 : (long long)bad[0];
         p->owner_runs = bad[1] == NOERR;
         p->faces_ok = bad[2] == NOERR;
-        rc = build_slots(h, p, c, f);
-        if (!rc) rc = build_halo(h, p, c, (long long)(bad[3] - INF_BITS) > 0);   // slot 3 starts there
+        const bool scattered = D == 2 && (long long)(bad[3] - INF_BITS) > 0;   // slot 3 starts there
+        rc = build_slots(h, p, c, f, widths);
+        if (!rc) rc = build_halo(h, p, c, scattered);
         if (!rc) rc = build_ghost_list(h, p, c);
     } while (0);
     if (rc) {
