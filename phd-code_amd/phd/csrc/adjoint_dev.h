@@ -575,7 +575,7 @@ PHD_HD inline void spatial_states_vjp(const double* com, double diff, const doub
 // cell's own and vol are in the ranges of quot_dev.h, so that the quotients by
 // r * vol may be taken with Shared.  (In the second walk the numerators are ldf *
 // area * (cfx -+ dr / 2), with ldf zero or in [2^-300, 2^300]: zero or in [2^-653,
-// 2^553], their quotients in [2^-905, 2^906].)  A distance or an ldf outside sends
+// 2^602], their quotients in [2^-955, 2^955].)  A distance or an ldf outside sends
 // the walk to the operators.  The quotients are 45 of a 3D entry's, and were three
 // quarters of the instructions.
 //

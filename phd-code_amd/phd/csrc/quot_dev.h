@@ -126,17 +126,20 @@ PHD_HD __forceinline__ bool zero_or_within(double x, double lo, double hi)
 // Operands of the gradient sums area * (d_dif cfx - d_sum dr / 2) / (r vol).
 // Coordinates (positions and face centroids) zero or >= 2^-100 are multiples of
 // 2^-152, so their differences and cfx are zero or >= 2^-153, and primitives zero or
-// >= 2^-290 give d_dif and d_sum / 2 zero or >= 2^-343.  Each product is zero or >=
-// 2^-495 and a multiple of 2^-548, so their difference is zero or >= 2^-548, and the
-// numerator, with an area zero or >= 2^-200, zero or >= 2^-748.  Above, it stays
-// below 2^(201 + 102 + 1 + 150) = 2^454.  The distance r = sqrt(sum dr^2) lies in
-// [2^-153, 2^102] unless zero, and r vol in [2^-353, 2^252]; so the quotients lie in
-// [2^-1000, 2^807].  (The limits leave room for cells of 2^-66 to 2^50 length units,
-// densities and pressures in any units, and velocities decaying ahead of a front.)
-PHD_HD __forceinline__ bool coord_ok(double x) { return zero_or_within(x, 0x1p-100, 0x1p100); }
-PHD_HD __forceinline__ bool prim_ok(double x) { return zero_or_within(x, 0x1p-290, 0x1p200); }
-PHD_HD __forceinline__ bool area_ok(double x) { return zero_or_within(x, 0x1p-200, 0x1p150); }
-PHD_HD __forceinline__ bool vol_ok(double x) { return within(x, 0x1p-200, 0x1p150); }
+// >= 2^-240 give d_dif and d_sum / 2 zero or >= 2^-293.  Each product is zero or >=
+// 2^-445 and a multiple of 2^-498, so their difference is zero or >= 2^-498, and the
+// numerator, with an area zero or >= 2^-200, zero or >= 2^-698.  Above, it stays
+// below 2^(151 + 151 + 1 + 150) = 2^453.  The distance r = sqrt(sum dr^2) lies in
+// [2^-153, 2^152] unless zero, and r vol in [2^-353, 2^302]; so the quotients lie in
+// [2^-1000, 2^806].  (The limits leave room for cells of 2^-66 to 2^50 length units,
+// densities and pressures in any units, and velocities decaying ahead of a front.
+// One upper limit for all: a pair of registers for each further one made the 2D
+// kernel spill, 12.15 -> 12.24 ms a pass of the 256-problem ensemble.)
+constexpr double SUM_MAX = 0x1p150;
+PHD_HD __forceinline__ bool coord_ok(double x) { return zero_or_within(x, 0x1p-100, SUM_MAX); }
+PHD_HD __forceinline__ bool prim_ok(double x) { return zero_or_within(x, 0x1p-240, SUM_MAX); }
+PHD_HD __forceinline__ bool area_ok(double x) { return zero_or_within(x, 0x1p-200, SUM_MAX); }
+PHD_HD __forceinline__ bool vol_ok(double x) { return within(x, 0x1p-200, SUM_MAX); }
 
 // densities and pressures, and the ratios of specific heats, that Shared takes
 PHD_HD __forceinline__ bool state_ok(double x) { return within(x, 0x1p-100, 0x1p100); }
