@@ -1107,8 +1107,9 @@ __global__ __launch_bounds__(BS) void k_face(phd_cells c, phd_faces f,
         // wave took 128^3 Sedov from 725 to 760 us), and keeps the operators.
         typename std::conditional<D == 2, Shared, Ieee>::type ar;
         if (D == 2) ar.ok = gas.shared;
-        face_flux<D, ORDER, SOLVER>(c, frec, rec, ld, m, i, j, fv, gas, dt_half, boost, gizmo, ar,
-                                    area, F);
+        if (D == 3 || gas.shared)
+            face_flux<D, ORDER, SOLVER>(c, frec, rec, ld, m, i, j, fv, gas, dt_half, boost, gizmo, ar,
+                                        area, F);
         if (D == 2 && !ar.ok) {
             // rows and record are read again through addresses of their own,
             // so that nothing is held for this across the first evaluation

@@ -76,8 +76,8 @@ struct Shared {
     {
         return {first ? a.b : b.b, first ? a.r : b.r};
     }
-    // a zero or |a| in [2^-760, 2^700], |a / b| in [2^-1000, 2^1000] or zero:
-    // the residual is then exact (a multiple of 2^-1074).  A smaller nonzero
+    // a zero or |a| in [2^-900, 2^700], |a / b| in [2^-1000, 2^1000] or zero:
+    // the residual is then exact (a multiple of 2^-1006).  A smaller nonzero
     // a is fine where only 1 + a/b is used.
     PHD_HD __forceinline__ double div(double a, Rcp c) const
     {
@@ -142,7 +142,7 @@ PHD_HD __forceinline__ bool area_ok(double x) { return zero_or_within(x, 0x1p-20
 PHD_HD __forceinline__ bool vol_ok(double x) { return within(x, 0x1p-200, SUM_MAX); }
 
 // densities and pressures, and the ratios of specific heats, that Shared takes
-PHD_HD __forceinline__ bool state_ok(double x) { return within(x, 0x1p-100, 0x1p100); }
+PHD_HD __forceinline__ bool state_ok(double x) { return within(x, 0x1p-132, 0x1p132); }
 inline bool shared_gamma(double gamma) { return gamma >= 1. + 0x1p-10 && gamma <= 64.; }
 
 } // namespace phd

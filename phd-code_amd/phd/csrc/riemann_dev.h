@@ -68,15 +68,16 @@ PHD_HD __forceinline__ double pow_b1(double x, double y)
 // and Toro eq. 10.68-10.70 wave speeds.  M: the arithmetic (quot_dev.h); rdl,
 // rdr its reciprocals of dl, dr.
 //
-// What Shared's checks give.  d, p in [2^-100, 2^100] and gamma in [1 + 2^-10,
-// 64] put c in [2^-34, 2^104]; |u| zero or in [2^-500, 2^100] bounds p* of the
-// first estimate by 2^310.  TRRS: (pl/pr)^z lies in [2^-100, 2^100], so the
-// numerators of u* are zero or >= 2^-760 and its divisor lies in [2^-205,
-// 2^140]; the two base quotients are only added to 1.  TSRS: every divisor lies
-// in [2^-211, 2^311], p* below 2^430.  The p* that results is checked, which
-// also sends NaN and overflow of the powers to Ieee.  p*/p - 1 is taken only
-// for p* > p, so the roots' arguments are >= 1.  sc: divisor < 0, checked with
-// its numerator.  max/min < 2 rounds to nearest as max < 2 min does for
+// What Shared's checks give.  d, p in [2^-132, 2^132] and gamma in [1 + 2^-10,
+// 64] put c in [2^-34, 2^135]; |u| zero or in [2^-500, 2^100] bounds p* of the
+// first estimate by 2^369.  TRRS: (pl/pr)^z lies in [2^-130, 2^130], the terms of
+// u*'s numerator are zero or >= 2^-765, so it is zero or >= 2^-817, and its divisor
+// lies in [2^-135, 2^165]; the two base quotients are only added to 1.  TSRS: every
+// divisor lies in [2^-253, 2^370], the numerator is zero or >= 2^-552, p* below
+// 2^518.  The p* that results is checked, which also sends NaN and overflow of the
+// powers to Ieee.  p*/p - 1 is taken only for p* > p, so the roots' arguments are
+// >= 1.  sc: divisor < 0, checked with its numerator, which it bounds by 2^402 (both
+// its terms are <= 0).  max/min < 2 rounds to nearest as max < 2 min does for
 // positive p: the quotient of floats below 2 min is at most 2 - 2^-52.
 template <class M>
 PHD_HD __forceinline__ void get_waves_m(double dl, double ul, double pl, double dr, double ur,

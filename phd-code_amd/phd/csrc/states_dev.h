@@ -133,7 +133,7 @@ PHD_HD __forceinline__ void spatial_states(const double* com, double diff, const
 // one side of PieceWiseLinear.add_temporal (reconstruction.pyx:1018-1072):
 // half-step primitive Euler predictor in the face frame.  Gradient groups:
 // d rho/dx_k = g[k], d v_q/dx_k = g[(1+q)D+k], d p/dx_k = g[(D+1)D+k].
-// Shared: numerators zero or >= 2^-700 over a density in [2^-100, 2^100].  One
+// Shared: numerators zero or >= 2^-700 over a density in [2^-132, 2^132].  One
 // that overflows leaves an infinite or NaN velocity, which the solver's check
 // of the normal velocity rejects, or none where the fallback restores S.
 template <int D, class M>
