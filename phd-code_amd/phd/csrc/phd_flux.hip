@@ -618,8 +618,8 @@ __attribute__((amdgpu_waves_per_eu(D == 2 ? 4 : 3))) void k_grad_sell(int n_cell
     // 2D AREPO: the first KC entries of each list keep their face centroid
     // in LDS from the gradient pass for the limiter pass ([entry][thread],
     // thread-private), so the limiter streams only the later slots again.
-    // 32 KB with the rows: four blocks still share a CU, as the 128 VGPRs
-    // allow (4096-problem step -0.8 %).  In 3D the 6 entries that would fit
+    // 40 KB with the rows and the halo: four blocks still share a CU, as the 128
+    // VGPRs allow (4096-problem step -0.8 %).  In 3D the 6 entries that would fit
     // beside three blocks changed nothing measurable.
     constexpr int KC = STAGE && LIM == PHD_LIMITER_AREPO && D == 2 ? 4 : 0;
     // 2D: the block's records leave through the same LDS, in natural order as
@@ -1102,7 +1102,7 @@ __global__ __launch_bounds__(BS) void k_face(phd_cells c, phd_faces f,
         }
     } else {
         // 2D: the quotients and roots are half of the instructions the kernel
-        // is bound by (4096-problem mix, 11.8 M faces: 535 -> 472 us).  3D: it
+        // is bound by (256-problem ensemble, 11.8 M faces: 535 -> 472 us).  3D: it
         // waits on its record gathers instead (1126 -> 962 VALU instructions a
         // wave took 128^3 Sedov from 725 to 760 us), and keeps the operators.
         typename std::conditional<D == 2, Shared, Ieee>::type ar;
@@ -1330,7 +1330,7 @@ __global__ __launch_bounds__(BS) void k_update_sell(phd_cells c, const double* _
 
 // The update from the caller's flux arrays and areas, three ways.
 //
-// Small meshes (below flux_stage_min windows) walk each cell's list entry by
+// Small meshes (below update_walk_max windows) walk each cell's list entry by
 // entry, k_update: their time is the chain perm -> slot -> face of the sliced
 // lists, and the CSR has one link less; blocks of 64 spread the cells over more
 // CUs (walk / sliced lists: 100^2 6.1 / 7.7 us, 256^2 9.3 / 12.2, 21^3 16.6 / 19.9,
@@ -1342,13 +1342,16 @@ __global__ __launch_bounds__(BS) void k_update_sell(phd_cells c, const double* _
 // there; the rest are gathered.  flux_cap rows and the update's own staging leave
 // four blocks a CU their LDS in 2D (800 rows; a window owns about 768 faces) and
 // two in 3D (1750 of about 2020).  Walk / staged: 400^2 15.8 / 16.7 us, 450^2 20.9 /
-// 17.9, 512^2 38.2 / 27.4; 36^3 30.0 / 32.2, 40^3 48.4 / 36.4, 48^3 137 / 42.
+// 17.9, 512^2 38.2 / 27.4; 36^3 30.0 / 32.2, 40^3 48.4 / 36.4, 48^3 137 / 42 (cells at
+// random: 450^2 105 / 101, 800^2 381 / 341, 40^3 119 / 105, 64^3 599 / 489).
 //
 // Larger ones with faces in any other order take the sliced lists, whose
-// entries load coalesced (walk / sliced, cells renumbered at random: 450^2 105 /
-// 101 us, 800^2 381 / 341, 40^3 119 / 105, 64^3 599 / 489; below the line 256^2 22.5
-// / 25.2, 21^3 16.1 / 19.7).
-template <int D> constexpr int flux_stage_min() { return D == 2 ? 700 : 256; }
+// entries load coalesced (walk / sliced, faces at random: 256^2 19.1 / 25.7 us, 400^2
+// 61.3 / 56.4, 512^2 118 / 107; 32^3 38.8 / 47.7, 36^3 61.6 / 55.2, 64^3 546 / 430).
+template <int D> constexpr int update_walk_max(bool owner_runs)
+{
+    return D == 2 ? (owner_runs ? 700 : 450) : owner_runs ? 256 : 200;
+}
 template <int D> constexpr int flux_cap() { return D == 2 ? 800 : 1750; }
 
 template <int D>
@@ -1920,7 +1923,7 @@ int launch_update_flux(phd_handle* h, phd_plan* p, const phd_cells* c, const Flu
 {
     if (c->n_cells == 0) return 0;
 #define UF(OR) k_update_flux<D, OR><<<xcd_grid(c->n_cells), PHD_BLOCK, 0, h->stream>>>(*c, p->n_faces, src, p->csr, p->off, p->perm, p->sbase, p->sfi, p->cinfo, h->d_err)
-    if (n_windows(c) < flux_stage_min<D>())
+    if (n_windows(c) < update_walk_max<D>(p->owner_runs))
         k_update<D><<<sched_grid<64, 1>(c->n_cells), 64, 0, h->stream>>>(*c, src, p->csr, p->off, h->d_err);
     else if (p->owner_runs) UF(1);
     else UF(0);

@@ -1,25 +1,31 @@
-"""The update from flux arrays on both sides of the line from which a window's
-faces are staged in LDS (700 windows of 256 cells in 2D, 256 in 3D), against the
-oracle, bit for bit: cells along the builder's curve, generators in random order
-(faces still in owner order, so that a window's cells have far neighbours and a
-face named by two windows is staged in one and gathered in the other), and cells
-renumbered after the faces (no owner order).  Some windows own more faces than are
-staged.  The fault it reports is the oracle's first."""
+"""The update from flux arrays on both sides of the line from which it leaves the
+plain walk of the lists (700 windows of 256 cells in 2D and 256 in 3D with faces in
+owner order, 450 and 200 otherwise), against the oracle, bit for bit: cells along
+the builder's curve; generators in random order (faces still in owner order, so
+that a window's cells have far neighbours and a face named by two windows is
+staged in one and gathered in the other); cells renumbered after the faces; and
+faces renumbered (no owner order: the sliced lists).  Some windows own more faces
+than are staged.  The fault it reports is the oracle's first."""
 import numpy as np
 import pytest
 import torch
 
 from parity import check_fields
 from test_gpu_cell_order import _renumber_cells
+from test_gpu_face_order import _owner_runs, _renumber
 
 pytestmark = pytest.mark.gpu
 
-MIN_WINDOWS = {2: 700, 3: 256}
+# windows from which the walk is left, with faces in owner order or not
+MIN_WINDOWS = {(2, True): 700, (3, True): 256, (2, False): 450, (3, False): 200}
+CASES = [(name, n, above, order) for name, n, above in
+         (("kh_2d", 410, False), ("kh_2d", 430, True), ("sedov_3d", 36, False), ("sedov_3d", 42, True))
+         for order in ("builder", "shuffled", "cells")] + \
+        [("kh_2d", 330, False, "faces"), ("kh_2d", 345, True, "faces"),
+         ("sedov_3d", 33, False, "faces"), ("sedov_3d", 37, True, "faces")]
 
 
-@pytest.mark.parametrize("order", ["builder", "shuffled", "renumbered"])
-@pytest.mark.parametrize("name,n,above", [("kh_2d", 410, False), ("kh_2d", 430, True),
-                                          ("sedov_3d", 36, False), ("sedov_3d", 42, True)])
+@pytest.mark.parametrize("name,n,above,order", CASES)
 def test_update_from_fluxes_both_sides(gpu, monkeypatch, name, n, above, order):
     from oracle import oracle
     from phd import problems
@@ -34,10 +40,12 @@ def test_update_from_fluxes_both_sides(gpu, monkeypatch, name, n, above, order):
         monkeypatch.setattr(problems, "jittered_lattice", shuffled)
     p = problems.PROBLEMS[name](n=n, seed=2)
     pc, mesh, dim = p.particles, p.mesh, p.dim
-    if order == "renumbered":
+    if order == "cells":
         _renumber_cells(p, seed=4)
+    if order == "faces":
+        _renumber(p, seed=11)
     windows = (pc.get_carray_size() + 255) // 256
-    assert (windows >= MIN_WINDOWS[dim]) == above, windows
+    assert (windows >= MIN_WINDOWS[dim, order != "faces"]) == above, windows
     rng = np.random.default_rng(n)
     for q, f in enumerate(pc.carray_named_groups["primitive"]):
         v = rng.uniform(0.5, 2.0, pc.get_carray_size())
@@ -45,7 +53,8 @@ def test_update_from_fluxes_both_sides(gpu, monkeypatch, name, n, above, order):
     p.eos.conservative_from_primitive(pc)
     a = problems.host_arrays(p)
     real = a["tag"] == 0
-    if order != "renumbered":       # owner order; windows own more than is staged (800, 1750)
+    assert _owner_runs(a) == (order != "faces")
+    if order in ("builder", "shuffled"):     # windows own more than is staged (800, 1750)
         assert (np.diff(a["pair_i"]) >= 0).all()
         assert np.bincount(a["pair_i"] // 256).max() > (800 if dim == 2 else 1750)
     flux = [rng.normal(0, 1, a["nf"]) for _ in range(dim + 2)]
