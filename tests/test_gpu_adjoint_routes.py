@@ -29,6 +29,12 @@ def _order(monkeypatch, how):
     monkeypatch.setattr(problems, "jittered_lattice", ordered)
 
 
+@pytest.mark.parametrize("name,n,pressure", [("kh_2d", 515, None), ("sedov_3d", 63, 1.0)])
+def test_reverse_of_large_meshes(gpu, name, n, pressure):
+    """Past 1024 windows, where the contributions are combined in blocks of 256."""
+    _check(gpu, name, n, pressure, 1, 1, None)
+
+
 @pytest.mark.parametrize("how", ["rows", "shuffled"])
 @pytest.mark.parametrize("name,n,pressure", [("kh_2d", 40, None), ("kh_2d", 185, None),
                                              ("sedov_3d", 12, 1.0), ("sedov_3d", 27, 1.0)])
