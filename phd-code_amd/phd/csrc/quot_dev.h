@@ -15,8 +15,10 @@
 // divisor's reciprocal once for all its numerators, gives the same correctly
 // rounded results (Markstein 1990: q + e r with q = a r, e = a - b q exact, is
 // the correctly rounded quotient) in 8 instructions per divisor and 3 per
-// numerator, 10 for a root.  A face of the 3D HLLC kernel has about 30
-// quotients and 8 roots, two thirds of its issue slots.
+// numerator, 10 for a root.  A 2D HLLC face has about 20 quotients and 8 roots,
+// half of its kernel's instructions; a 2D gradient entry divides 8 numerators by
+// one divisor, a 3D entry 15.  (The 3D face kernel waits on its gathers instead and
+// keeps the operators.)
 //
 // Shared keeps one flag: `ok` falls when an operand leaves the ranges for
 // which the comment at the place shows the sequence to be exact, and the
