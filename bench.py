@@ -46,7 +46,7 @@ VALU_WAVE_INSTR_PER_S = 256 * 4 * 2.4e9 / 4
 CSRC = os.path.join(ROOT, "phd-code_amd", "phd", "csrc")
 PROFILES = os.path.join(ROOT, "profiles")
 # bench stage -> rocprofv3 kernel name of the 3D kernel it launches
-KERNEL_NAMES = {"gradients": "k_grad_sell<3, 0, 256, 1, 5>",
+KERNEL_NAMES = {"gradients": "k_grad_sell<3, 0, 256, 1, 5, 1>",
                 "face_flux": "k_face<3, 1, 1, 2, 0, 256, 1, 3>",
                 "update": "k_update_sell<3, 256, 1, 1>", "ghost_gradients": "k_ghost_rec<3>",
                 "epilogue": "k_ghost_refresh_eos<3, 0>"}
